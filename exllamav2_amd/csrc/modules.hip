@@ -140,6 +140,7 @@ struct QMoEMLP
     bool lean_rows_ok[LEAN_MAX_M + 1]; LeanGroupPlan lean_gu_r[LEAN_MAX_M + 1], lean_dn_r[LEAN_MAX_M + 1];      // 2-4 rows: one launch over all experts each (the reference's fused form covers <= 4 rows, q_mlp.cu:316-436)
     // more than 16 rows: all experts in one launch per projection (qgemm_tile.hip); device tables made here
     bool tile_ok, tile_pair; QMatDev* tile_mats; const u16** tile_invperms;      // [E][w1, w3, w2]; [E] w2's packed order (null: natural order)
+    bool down_bias;                             // some expert's w2 has a bias
     bool lean_sum_ok; LeanGroupPlan lean_dn2;      // top-2: both selected experts' down projections as ONE pair launch that adds the weighted sum to x (no combine launch)
 };
 
@@ -229,11 +230,12 @@ KERNEL void __launch_bounds__(256) moe_combine_kernel(f16* x, const f16* part, c
     }
 }
 
-// 2 .. 64 rows (qgemm_skinny.hip: experts): x[r, :] += sum over the row's experts of weight * sum over the K splits of its slot's partial
-// tile, fp32 in expert and split order, one rounding; published like moe_combine_kernel does.  A row's slot in an expert is the number of
-// rows before it that chose the expert (a ballot per expert).
+// 2 .. 64 rows (qgemm_skinny.hip: experts): x[r, :] += sum over the row's experts of weight * (sum over the K splits of its slot's partial
+// tile + down's bias), fp32 in expert and split order, one rounding; published like moe_combine_kernel does.  A row's slot in an expert is
+// the number of rows before it that chose the expert (a ballot per expert).  `mats`: the experts' matrices [E][w1, w3, w2], null where no
+// w2 has a bias (nothing to look up)
 KERNEL void __launch_bounds__(256) moe_sum_slots_kernel(f16* x, const f32x4* part, const f16* weights, int rows, int hidden, int E, int RB, int groups,
-                                                       int ks, const MoeChainOut co)
+                                                       int ks, const QMatDev* mats, const MoeChainOut co)
 {
     SHARED float sq_part[4];
     const int row = bid_y(), o = bid_x() * 256 + tid(), lane = lane_id();
@@ -255,6 +257,12 @@ KERNEL void __launch_bounds__(256) moe_sum_slots_kernel(f16* x, const f32x4* par
         const f32x4* p = part + (((((size_t)e * groups + grp) * ks * 4 + wv) * RB + (slot >> 4)) * 2 + ct) * 64 + j4 * 16 + (slot & 15);
         f32x4 a = p[0], b = p[16];
         for (int z = 1; z < ks; z++) { a += p[(size_t)z * 4 * RB * 2 * 64]; b += p[(size_t)z * 4 * RB * 2 * 64 + 16]; }
+        const f16* const bias = mats ? mats[3 * e + 2].bias : nullptr;
+        if (bias)
+        {
+            #pragma unroll
+            for (int k = 0; k < 4; k++) { a[k] += (float)bias[n + k]; b[k] += (float)bias[n + 4 + k]; }
+        }
         #pragma unroll
         for (int k = 0; k < 4; k++) { acc[k] = fmaf(w, a[k], acc[k]); acc[4 + k] = fmaf(w, b[k], acc[4 + k]); }
     }
@@ -583,7 +591,8 @@ static int moe_forward_slots(QMoEMLP* m, f16* x, const f16* xg, int rows, const 
     { const int rc = qgemm_skinny_experts_launch(d, inter, gptq, stream); if (rc) return rc; }
     if (ENV_SET("EXL2_DEBUG_ROUTE")) fprintf(stderr, "q_moe_mlp route: slots rows=%d experts=%d splits=%d\n", rows, E, d.ks);
     LAUNCH(moe_sum_slots_kernel, dim3((unsigned)((hidden / 8 + 255) / 256), (unsigned)rows), dim3(256), 0, stream,
-           x, (const f32x4*)d.part, (const f16*)m->temp_logits, rows, hidden, E, rb, d.groups, d.ks, co);
+           x, (const f32x4*)d.part, (const f16*)m->temp_logits, rows, hidden, E, rb, d.groups, d.ks,
+           (const QMatDev*)(m->down_bias ? m->tile_mats : nullptr), co);
     HIP_TRY(hipGetLastError());
     if (npart_out) *npart_out = co.xp ? (hidden / 8 + 255) / 256 : 0;
     return EXL2_OK;
@@ -677,6 +686,7 @@ int exl2_make_q_moe_mlp(void** handle, const void* layernorm, const void* layern
         for (int i = 0; i < num_experts; i++) { all[2 * i] = m->w1[i]; all[2 * i + 1] = m->w3[i]; }
         m->group_ok = num_experts <= 16 && same_perm(all, 2 * num_experts) && hidden_ok(m);
     }
+    for (int e = 0; e < num_experts; e++) if (m->w2[e]->dev.bias) m->down_bias = true;
     moe_plan_lean(m);
     { const int rc = moe_plan_tile(m); if (rc) { exl2_free_q_moe_mlp(m); return rc; } }
     *handle = m;

@@ -30,23 +30,25 @@ def test_moe_route(be, experts, topk):
     assert np.allclose(got.astype(np.float32).sum(-1), 1.0, atol=2e-3)
 
 
-def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31, spec_up=None, spec_dn=None, gate_scale=0.3, spec_w3=None, max_rows=128):
-    """one sparse-MoE block (q_moe_mlp_forward_) against the oracle's composition: routing mask, weighted expert sum into the residual"""
+def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31, spec_up=None, spec_dn=None, gate_scale=0.3, spec_w3=None, max_rows=128, bias=0.0):
+    """one sparse-MoE block (q_moe_mlp_forward_) against the oracle's composition: routing mask, weighted expert sum into the residual.
+    bias: root mean square of the biases of down (gate and up: a quarter of it), none at 0"""
     from tests.util import exl2_to_torch
     rng = np.random.default_rng(seed)
     spec_up = spec_up or [(5, 32, 32), (4, 32, hidden - 32)]
     spec_dn = spec_dn or [(5, 32, 64), (4, 64, inter - 64)]
-    keep, handles, refs = [], {"w1": [], "w2": [], "w3": []}, {"w1": [], "w2": [], "w3": []}
+    keep, handles, refs, biases = [], {"w1": [], "w2": [], "w3": []}, {"w1": [], "w2": [], "w3": []}, {"w1": [], "w2": [], "w3": []}
     shared = rng.permutation(hidden).astype(np.int32)
     for e in range(E):
         for name, (k, n, spec) in (("w1", (hidden, inter, spec_up)), ("w3", (hidden, inter, spec_w3 or spec_up)), ("w2", (inter, hidden, spec_dn))):
             t = OX.synth_exl2(k, n, spec, seed=100 + 3 * e + len(name) + ord(name[1]), act_order=True)
+            if bias: t["bias"] = (np.random.default_rng([seed, e, k, n]).standard_normal(n) * (bias if name == "w2" else bias / 4)).astype(F16)
             if shared_perm and name != "w2":
                 t["q_invperm"] = shared.copy()
             ref = OX.exl2_reconstruct(t)
             w = exl2_to_torch(be, t)
             h = be.ext.make_q_matrix_from_dict(w, None)
-            keep.append(w); handles[name].append(h); refs[name].append(ref)
+            keep.append(w); handles[name].append(h); refs[name].append(ref); biases[name].append(t.get("bias"))
     norm_w = (1.0 + 0.1 * rng.standard_normal(hidden)).astype(F16)
     gate = (rng.standard_normal((E, hidden)) * gate_scale).astype(F16)
     x = rng.standard_normal((rows, hidden)).astype(F16)
@@ -82,10 +84,10 @@ def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31
     for e in range(E):
         sel = np.nonzero(mask[:, e])[0]
         if len(sel) == 0: continue
-        g = OX.gemm_ref(xn[sel], refs["w1"][e], exact=True).astype(F16)
-        u = OX.gemm_ref(xn[sel], refs["w3"][e], exact=True).astype(F16)
+        g = OX.gemm_ref(xn[sel], refs["w1"][e], bias=biases["w1"][e], exact=True).astype(F16)
+        u = OX.gemm_ref(xn[sel], refs["w3"][e], bias=biases["w3"][e], exact=True).astype(F16)
         a = OM.silu_mul(g, u)
-        d = OX.gemm_ref(a, refs["w2"][e], exact=True)
+        d = OX.gemm_ref(a, refs["w2"][e], bias=biases["w2"][e], exact=True)
         want[sel] += d * wts[sel, e].astype(np.float64)[:, None]
     tol = np.abs(want) * 2.0 ** -8 + 6e-3                   # E sequential fp16 accumulations into the residual
     assert np.all((np.abs(got - want) <= tol)[clear]), float(np.abs(got - want)[clear].max())
@@ -137,6 +139,15 @@ def test_moe_slots(be, rows, E, topk, hidden, inter, ks, capfd, monkeypatch):
     monkeypatch.setenv("EXL2_SKINNY_EXPERT_KS", str(ks))
     _moe_case(be, rows, True, E=E, topk=topk, hidden=hidden, inter=inter, gate_scale=0.6, spec_dn=[(5, 32, 64), (3, 32, inter - 64)], max_rows=160)
     assert f"route: slots rows={rows} experts={E} splits={min(ks, 1 - (64 - inter) // 128)}" in capfd.readouterr().err
+
+
+@pytest.mark.parametrize("rows,ks", [(2, 1), (5, 2), (16, 1), (17, 2), (64, 2), (65, 0)])
+def test_moe_experts_with_biases(be, rows, ks, capfd, monkeypatch):
+    """Biases of all three projections, large against the tolerance, at row counts of the slots route (K splits: added once) and of the tiles."""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    if ks: monkeypatch.setenv("EXL2_SKINNY_EXPERT_KS", str(ks))
+    _moe_case(be, rows, True, gate_scale=0.6, bias=2.0)
+    assert ("route: slots" if ks else "route: tiles") in capfd.readouterr().err
 
 
 def test_moe_model_forward(be):
