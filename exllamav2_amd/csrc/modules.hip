@@ -513,7 +513,8 @@ static void moe_plan_lean(QMoEMLP* m)
         if (qgemv_lean_group_plan(ins, E, scale, 1, &m->lean_dn_r[r], E, 1) != 0) { qgemv_lean_group_free(&m->lean_gu_r[r]); continue; }
         m->lean_rows_ok[r] = true;
     }
-    if (m->num_experts_per_token == 2 && !getenv("EXL2_MOE_NO_SUM_PLAN"))
+    // (the summing launch's epilogue adds no bias: experts with one take the two launches and the combine launch)
+    if (m->num_experts_per_token == 2 && !m->down_bias && !getenv("EXL2_MOE_NO_SUM_PLAN"))
     {
         for (int e = 0; e < E; e++)
         {

@@ -150,6 +150,14 @@ def test_moe_experts_with_biases(be, rows, ks, capfd, monkeypatch):
     assert ("route: slots" if ks else "route: tiles") in capfd.readouterr().err
 
 
+@pytest.mark.parametrize("topk", [1, 2])
+def test_moe_one_row_with_biases(be, topk, capfd, monkeypatch):
+    """One row on the lean kernel with biases: the launch that sums two experts' down projections has none, so the combine launch follows."""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    _moe_case(be, 1, True, topk=topk, hidden=256, inter=512, bias=2.0)
+    assert "route: lean rows=1" in capfd.readouterr().err
+
+
 def test_moe_model_forward(be):
     """Mixtral-style model through the ordinary ExLlamaV2 loop (config.num_experts > 0): prefill + decode run, logits are
     finite, two identical sequences in a batch produce identical rows, and the sparse MLP of layer 0 applied by hand to
