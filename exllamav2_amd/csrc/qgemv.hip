@@ -277,15 +277,15 @@ KERNEL void __launch_bounds__(1024) qgemv_kernel(const GemvArgs args)
         const int n = tile * 16 + c;
         const int grow = row0 + row;
         bool skip = false;
+        if (m.bias) v += (float)m.bias[n];
         if (job.r_weights)
         {
             const f16 rw = job.r_weights[(size_t)grow * job.r_stride];
             if (as_u16(rw) == 0) skip = true;                       // q_gemm_kernel.cuh:189-200: zero weight -> no-op
-            if (job.mul_r_weights) v *= (float)rw;
+            if (job.mul_r_weights) v *= (float)rw;                  // the expert's whole output, its bias with it
         }
         if (!skip)
         {
-            if (m.bias) v += (float)m.bias[n];
             f16* cp = job.c + (size_t)grow * job.ldc + (job.c_invperm ? (int)job.c_invperm[n] : n);
             if (job.c_mode == C_ACCUM) v += (float)*cp;
             *cp = (f16)v;

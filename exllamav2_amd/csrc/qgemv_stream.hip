@@ -340,15 +340,15 @@ KERNEL void __launch_bounds__(1024) qgemv_stream_kernel(const StreamArgs args)
         for (int w = 0; w < S; w++) v += red[((slot * S + w) * 16 + row) * 16 + c];
         const int n = tl * 16 + c;
         bool skip = false;
+        if (m.bias) v += (float)m.bias[n];
         if (job.r_weights)
         {
             const f16 rw = job.r_weights[(size_t)row * job.r_stride];
             if (as_u16(rw) == 0) skip = true;                       // q_gemm_kernel.cuh:189-200
-            if (job.mul_r_weights) v *= (float)rw;
+            if (job.mul_r_weights) v *= (float)rw;                  // the expert's whole output, its bias with it
         }
         if (!skip)
         {
-            if (m.bias) v += (float)m.bias[n];
             f16* cp = job.c + (size_t)row * job.ldc + (job.c_invperm ? (int)job.c_invperm[n] : n);
             if (job.c_mode == C_ACCUM) v += (float)*cp;
             *cp = (f16)v;
@@ -518,15 +518,15 @@ KERNEL void __launch_bounds__(1024) qgemv_phased_kernel(const PhasedArgs args)
         for (int w = 0; w < S; w++) v += red[((slot * S + w) * 16 + row) * 16 + c];
         const int n = tl * 16 + c;
         bool skip = false;
+        if (m.bias) v += (float)m.bias[n];
         if (job.r_weights)
         {
             const f16 rw = job.r_weights[(size_t)row * job.r_stride];
             if (as_u16(rw) == 0) skip = true;
-            if (job.mul_r_weights) v *= (float)rw;
+            if (job.mul_r_weights) v *= (float)rw;                  // the expert's whole output, its bias with it
         }
         if (!skip)
         {
-            if (m.bias) v += (float)m.bias[n];
             f16* cp = job.c + (size_t)row * job.ldc + (job.c_invperm ? (int)job.c_invperm[n] : n);
             if (job.c_mode == C_ACCUM) v += (float)*cp;
             *cp = (f16)v;

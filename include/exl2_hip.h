@@ -48,7 +48,7 @@ int exl2_q_matrix_info(void* handle, int* height, int* width, int* groups, int* 
 int exl2_reconstruct(void* handle, void* out, void* stream);
 /* gemm_half_q_half (ext_qmatrix.cpp:213-247 -> gemm_half_q_half_cuda cuda/q_gemm.cu:201-313): c[M,N] (+)= a[M,K] W
  * (+ bias).  clear = 0 accumulates into c (residual).  r_weights: optional MoE routing weights half[M, r_weights_stride]
- * (zero weight -> row skipped; mul_r_weights -> result scaled; cuda/q_gemm_kernel.cuh:189-200,553-558). */
+ * (zero weight -> row skipped; mul_r_weights -> a W + bias scaled; cuda/q_gemm_kernel.cuh:189-200,553-558). */
 int exl2_gemm_half_q_half(const void* a, void* handle, void* c, int size_m, int clear,
                           const void* r_weights, int r_weights_stride, int mul_r_weights, void* stream);
 /* make_group_map (ext_qmatrix.cpp:341-361), host only: returns number of uint16 written (2K) or < 0 */

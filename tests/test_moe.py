@@ -158,6 +158,15 @@ def test_moe_one_row_with_biases(be, topk, capfd, monkeypatch):
     assert "route: lean rows=1" in capfd.readouterr().err
 
 
+@pytest.mark.parametrize("rows,shared_perm,env", [(1, False, None), (3, False, None), (21, False, None), (5, True, "EXL2_MOE_NO_GROUP"), (16, True, "EXL2_MOE_NO_GROUP"),
+                                                  (9, False, "EXL2_GEMV_PHASED"), (4, False, "EXL2_GEMV_GENERIC")])
+def test_moe_experts_with_biases_launch_by_launch(be, rows, shared_perm, env, monkeypatch):
+    """The same on the kernels that take the routing weights of one expert per job (streaming, phased, generic): down's bias is weighted like
+    the product."""
+    if env: monkeypatch.setenv(env, "1")
+    _moe_case(be, rows, shared_perm, gate_scale=0.6, bias=2.0)
+
+
 def test_moe_model_forward(be):
     """Mixtral-style model through the ordinary ExLlamaV2 loop (config.num_experts > 0): prefill + decode run, logits are
     finite, two identical sequences in a batch produce identical rows, and the sparse MLP of layer 0 applied by hand to
