@@ -403,6 +403,24 @@ def test_flash_prefill_nan_scores(be, s, past):
     assert np.all(np.abs(be.n(out).astype(np.float32) - want) <= _attn_tol(want))
 
 
+@pytest.mark.parametrize("s, past", [(200, 400), (20, 900)])
+@pytest.mark.parametrize("amp", [64.0, 4000.0, 8000.0, 50000.0])
+def test_flash_prefill_large_scores(be, s, past, amp):
+    """Scores up to 2.8e10, whose rounding steps (2048) are beyond the exponential's range: a tile without a mask must not take the fused
+    exponent there.  Every query row equals one key and the rest are far below: the output is that key's value (half an fp16 step of the
+    probability, half a step of the result)."""
+    rng = np.random.default_rng(int(amp))
+    hd, nh, total = 128, 2, past + s
+    signs = lambda n: (rng.integers(0, 2, size=(1, n, nh, hd)) * 2 - 1) * amp
+    q, k, v = signs(s).astype(F16), signs(total).astype(F16), rng.standard_normal((1, total, nh, hd)).astype(F16)
+    at = rng.permutation(past)[:s]
+    k[:, at] = q
+    out = torch.full((1, s, nh, hd), 77.0, dtype=torch.float16, device=be.device)
+    assert be.ext.flash_prefill(be.t(q), be.t(k), be.t(v), out, None, None, len_const=past, len_offset=s)
+    want = v[:, at].astype(np.float32)
+    assert np.all(np.abs(be.n(out).astype(np.float32) - want) <= np.abs(want) * 2.0 ** -10 + 2.0 ** -24)
+
+
 @pytest.mark.parametrize("be", [pytest.param("hip", marks=pytest.mark.gpu)], indirect=True)
 def test_flash_prefill_captured_without_scratch(be):
     """A graph captured on a stream that holds no workspace yet cannot get one: the keys are not split there, and every replay is right."""
