@@ -206,8 +206,8 @@ KERNEL void __launch_bounds__(FP_WAVES * 64, FP_OCC) flash_prefill_kernel(const 
         }
         // mask + online softmax for column qi of each query block (lane holds keys k0 + 16 blk + 4 g + r).  A tile that every row of the wave
         // sees whole (all but the last one or two of a causal block) needs no mask: per score one maximum, one fused multiply-add into
-        // the exponent, the exponential and the sum.  (An infinite or NaN score shows in the sum, and so does a maximum so large -- 2^28 on --
-        // that its rounding, which the fused exponent of its own key keeps, is no small step: such a tile goes the general way.)
+        // the exponent, the exponential and the sum.  (A NaN score shows in the sum.  The fused exponent of the largest key is the rounding of the
+        // maximum and not 0: it scales the row's probabilities alike, by 1/e to e up to 2^24.  Tiles beyond either go the general way.)
         // Causal 8 x 2048 rows of 32 heads of 128: 755 us with the mask and the rescale in every tile, 685 so (0.40 PFLOP/s over the visible scores).
         f16x8 pb[RPW][NBLK / 2];                     // B operands: 32 keys each = {block 2n keys 4g..4g+3, block 2n+1 keys 4g..4g+3}
         float alpha[RPW];
@@ -234,7 +234,7 @@ KERNEL void __launch_bounds__(FP_WAVES * 64, FP_OCC) flash_prefill_kernel(const 
                     p_sum += p;
                     pb[n][e / 8][e % 8] = (f16)p;
                 }
-                done = wave_ballot(!(p_sum <= 8.0f * NBLK)) == 0;             // (4 NBLK probabilities of at most 1, and room for that rounding)
+                done = wave_ballot(!(p_sum >= 0.0f) || !(fabsf(m_new) <= 16777216.0f)) == 0;
                 if (done)
                 {
                     alpha[n] = fast_exp(m_run[n] - m_new);

@@ -404,7 +404,7 @@ def test_flash_prefill_nan_scores(be, s, past):
 
 
 @pytest.mark.parametrize("s, past", [(200, 400), (20, 900)])
-@pytest.mark.parametrize("amp", [64.0, 4000.0, 8000.0, 50000.0])
+@pytest.mark.parametrize("amp", [64.0, 1000.0, 1200.0, 1300.0, 4000.0, 8000.0, 50000.0])
 def test_flash_prefill_large_scores(be, s, past, amp):
     """Scores up to 2.8e10, whose rounding steps (2048) are beyond the exponential's range: a tile without a mask must not take the fused
     exponent there.  Every query row equals one key and the rest are far below: the output is that key's value (half an fp16 step of the
