@@ -402,7 +402,7 @@ int exl2_flash_prefill_ex(const void* q, const void* k_cache, const void* v_cach
 {
     EXL2_REQUIRE(window_left < 0 || causal, "flash_prefill: a sliding window needs causal attention");
     EXL2_REQUIRE(q && k_cache && v_cache && out, "flash_prefill: null argument");
-    EXL2_REQUIRE(num_kv_heads > 0 && num_heads % num_kv_heads == 0, "flash_prefill: heads %d not a multiple of kv heads %d", num_heads, num_kv_heads);
+    EXL2_REQUIRE(num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0, "flash_prefill: heads %d not a multiple of kv heads %d", num_heads, num_kv_heads);
     if (batch <= 0 || q_len <= 0) return EXL2_OK;
     if (!(head_dim == 64 || head_dim == 128 || head_dim == 256)) return 1;
     FlashArgs a;

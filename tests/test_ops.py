@@ -421,6 +421,15 @@ def test_flash_prefill_large_scores(be, s, past, amp):
     assert np.all(np.abs(be.n(out).astype(np.float32) - want) <= np.abs(want) * 2.0 ** -10 + 2.0 ** -24)
 
 
+@pytest.mark.parametrize("be", ["emu"], indirect=True)
+def test_flash_prefill_without_heads_is_refused(be):
+    """No heads: an error, before the launch's shape is worked out (the estimate of the key splits divides by the number of workgroups)."""
+    t = torch.zeros(4096, dtype=torch.float16)
+    for heads in (0, -2):
+        with pytest.raises(Exception, match="heads"):
+            be.ext.lib.check(be.ext.lib.exl2_flash_prefill(t.data_ptr(), t.data_ptr(), t.data_ptr(), t.data_ptr(), None, None, 1, 2, heads, 1, 64, 0, 0, 10, 2, 0.125, 1, None))
+
+
 @pytest.mark.parametrize("be", [pytest.param("hip", marks=pytest.mark.gpu)], indirect=True)
 def test_flash_prefill_captured_without_scratch(be):
     """A graph captured on a stream that holds no workspace yet cannot get one: the keys are not split there, and every replay is right."""
