@@ -588,7 +588,7 @@ static int launch_one(const MfArgs& p, void* stream)
 {
     g_last_route[0] = p.M; g_last_route[1] = MT; g_last_route[2] = WPRE ? 1 : 0; g_last_route[3]++;
     const int nb_m = (p.M + 32 * MT - 1) / (32 * MT);
-    if (getenv("EXL2_PREFILL_TRACE")) fprintf(stderr, "[qgemm_mfma] M=%d K=%d column blocks=%d splits=%d MT=%d gptq=%d\n", p.M, p.job[0].m.K, p.block0[MF_MAX_JOBS], p.ks, MT, (int)GPTQ);
+    if (getenv("EXL2_PREFILL_TRACE")) fprintf(stderr, "[qgemm_mfma] M=%d K=%d column blocks=%d splits=%d MT=%d gptq=%d pre=%d\n", p.M, p.job[0].m.K, p.block0[MF_MAX_JOBS], p.ks, MT, (int)GPTQ, (int)WPRE);
     LAUNCH((qgemm_mfma_kernel<GPTQ, MT, WPRE>), dim3((unsigned)(p.block0[MF_MAX_JOBS] * nb_m * p.ks)), dim3(MF_THREADS), 0, stream, p);
     if (p.ks > 1) LAUNCH((mf_reduce_kernel<MT>), dim3((unsigned)(p.block0[MF_MAX_JOBS] * nb_m * (8 * MT * 4 * 64 / 256))), dim3(256), 0, stream, p);
     return EXL2_OK;
@@ -632,12 +632,14 @@ int qgemm_mfma_launch(const PrefillArgs* pas, int n, bool gptq, void* stream)
     // at 333 rows (48 tiles of 128 rows) 71.6 / 41.3 us in four, 11008 x 4096 161.7 / 79 us in four, 4096 x 11008 at 160 rows 79.8 / 64
     // us in two; one launch for q | k | v and for gate | up on top: a 333-token prompt of 32 7B layers 19.9 -> 12.3 ms.
     const int cus = device_cus();
-    // (many rounds anyway: a launch per matrix keeps one matrix' fragments in the memory-side cache, 0.2 % at 16384 rows)
-    if (n > 1 && (long)blocks * ((M + 255) / 256) >= 8L * cus)
+    auto one_by_one = [&]() -> int
     {
         for (int i = 0; i < n; i++) { const int rc = qgemm_mfma_launch(pas + i, 1, gptq, stream); if (rc) return rc; }
         return EXL2_OK;
-    }
+    };
+    // (many rounds anyway: a launch per matrix keeps one matrix' fragments in the memory-side cache, 0.2 % at 16384 rows.  A matrix of more
+    // sections than the arguments name can neither split K nor have its fragments made: the others are not held to that)
+    if (n > 1 && ((long)blocks * ((M + 255) / 256) >= 8L * cus || (!runs && supers_max > 0))) return one_by_one();
     int mt = 8, ks = 1;
     {
         const double steps = 2.0 * (supers_max > 0 ? supers_max : (K + SUPER_ROWS - 1) / SUPER_ROWS);
@@ -683,12 +685,8 @@ int qgemm_mfma_launch(const PrefillArgs* pas, int n, bool gptq, void* stream)
         size_t cap = (size_t)1 << 30;
         if (const char* e = getenv("EXL2_PREFILL_WPRE_MAX_BYTES")) cap = (size_t)strtoull(e, nullptr, 10);
         if (cap >= ((size_t)1 << 31)) cap = ((size_t)1 << 31) - 1;      // (the W stages are filled by buffer loads: a 2 GB window)
-        if (bytes > cap && n > 1)
-        {
-            for (int i = 0; i < n; i++) { const int rc = qgemm_mfma_launch(pas + i, 1, gptq, stream); if (rc) return rc; }
-            return EXL2_OK;
-        }
         if (bytes <= cap) buf = prefill_scratch_try(bytes, stream, 1);
+        if (!buf && n > 1) return one_by_one();                           // (less at a time may fit)
         if (buf)
         {
             for (int i = 0; i < n; i++) p.job[i].wfrag = (const u8*)buf + at[i];

@@ -275,6 +275,30 @@ def test_prefill_matrices_over_the_same_rows_share_a_launch(be, monkeypatch):
     assert outs[3] - outs[1] == 3 * cfg.num_hidden_layers
 
 
+def test_prefill_matrix_of_many_sections_beside_one_of_few(be, capfd, monkeypatch):
+    """gate in one section, up in more than a kernel's argument block names: up decodes inside its product, gate's weights are decoded ahead as
+    they are alone -- the two do not share a launch."""
+    from exllamav2_amd.ext import none_tensor
+    monkeypatch.setenv("EXL2_PREFILL_WPRE_MIN_ROWS", "1")
+    monkeypatch.setenv("EXL2_PREFILL_TRACE", "1")
+    k, n, m = 448, 256, 130
+    tg, rg, wg, hg = make_exl2(be, k, n, [(4, 32, k)], seed=51, act_order=False)
+    tu, ru, wu, hu = make_exl2(be, k, n, [(b, 32, 32) for b in (4, 3) * 7], seed=52, act_order=False)
+    td, rd, wd, hd = make_exl2(be, n, k, [(4, 32, n)], seed=53, act_order=False)
+    rows = lambda w: torch.zeros((m, w), dtype=torch.float16, device=be.device)
+    ta, tb = rows(n), rows(n)
+    mlp = be.ext.make_q_mlp(none_tensor, none_tensor, True, 1e-5, hg, hu, hd, none_tensor, ta, tb, none_tensor, m, False, True, none_tensor, none_tensor, False, False)
+    x = (np.random.default_rng(54).standard_normal((m, k)) * 0.5).astype(np.float16)
+    xt = be.t(x)
+    be.ext.q_mlp_forward_(mlp, xt)
+    assert [l[-1] for l in capfd.readouterr().err.splitlines() if "[qgemm_mfma]" in l] == ["1", "0", "1"]
+    g, u = OX.gemm_ref(x, rg).astype(np.float64), OX.gemm_ref(x, ru).astype(np.float64)
+    want = OX.gemm_ref((g / (1 + np.exp(-g)) * u).astype(np.float16), rd, exact=True) + x
+    assert np.all(np.abs(be.n(xt).astype(np.float64) - want) <= np.abs(want) * 2.0 ** -8 + 6e-3)
+    be.ext.free_q_mlp(mlp)
+    for h in (hg, hu, hd): be.ext.free_q_matrix(h)
+
+
 def test_prefill_predecode_scratch_cap_falls_back(be, monkeypatch):
     """The weights-decoded-once route needs K * N * 2 bytes of scratch; above the cap (or when the allocation fails) the call must
     run with the decode inside the GEMM instead of failing -- same result bit for bit (same decoders, same rounding)."""
