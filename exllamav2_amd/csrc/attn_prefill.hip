@@ -24,6 +24,8 @@
 // Bound: MFMA (2 * s * T * hd FLOP per head) -- 16 MFMAs per 32 keys per wave against ~60 VALU ops of softmax.
 #include "hw.h"
 #include "errors.h"
+#include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 f16* prefill_scratch_try(size_t bytes, void* stream, int kind);       // qgemm_prefill.hip: scratch per (device, stream); kind 4 is this file's
@@ -416,9 +418,13 @@ int exl2_flash_prefill_ex(const void* q, const void* k_cache, const void* v_cach
     a.len_const = len_const; a.len_offset = len_offset; a.scale = softmax_scale; a.causal = causal;
     FlashWS w; w.window_left = window_left; w.softcap = softcap > 0.0f ? softcap : 0.0f;
     const bool ws = w.window_left >= 0 || w.softcap > 0.0f;
-    // Key splits where the query blocks leave CUs idle and the host knows the lengths: two tiles of 64 keys each at least, one round of
-    // workgroups (two per CU).  37 rows behind 600 keys are 32 workgroups that walk ten tiles one
-    // after the other: 25 us; in five splits, merging launch included, 14 (the 32 layers of such a turn 4.80 -> 4.44 ms).
+    // Key splits where the query blocks leave CUs idle and the host knows the lengths: one round of workgroups (two per CU), two tiles of 64
+    // keys for the longest query block each at least, and only where an estimate says that they pay: that block's tiles (us each alone on a CU,
+    // 1.3 of it with two workgroups) against the merging launch (2 us, 0.5 per split, 0.45 per MB of partial results).
+    // Whole calls on the MI355X, us, in one split | in the rule's number: 32 heads of 128, 37 rows behind 600 keys 25.3 | 13.8 in five, 200
+    // behind 600 32.2 | 22.7 in six, 333 behind 2000 83.1 | 42.3 in five; 64 heads, 37 behind 8000 267 | 59.6 in eight.  Where it does not:
+    // 333 rows of a prompt's start 17.0 (three splits: 23.1), 500 rows 22.3 (four: 25.6).  Of 310 shapes (8 - 64 heads of 64, 128, 256, 4 -
+    // 1024 rows behind 0 - 8000 keys) none that it splits is slower for it, one that it leaves (31.5) would gain 1.8
     a.splits = 1;
     if (!ws && !cache_seqlens)
     {
@@ -429,9 +435,16 @@ int exl2_flash_prefill_ex(const void* q, const void* k_cache, const void* v_cach
         if (n > 8) n = 8;
         if (n >= 3)                                           // (two splits gain less than the merging launch costs)
         {
-            a.part = (float*)prefill_scratch_try((size_t)batch * n * q_len * num_heads * (head_dim + 2) * sizeof(float), stream, 4);
-            if (a.part) a.splits = n;
+            const size_t bytes = (size_t)batch * n * q_len * num_heads * (head_dim + 2) * sizeof(float);
+            const double tile = head_dim == 64 ? 1.55 : head_dim == 128 ? 2.05 : 9.0;
+            const double split = tile * (wgs * n > 256 ? 1.3 : 1.0) * ((tiles + n - 1) / n) + 2.0 + 0.5 * n + 0.45e-6 * (double)bytes;
+            if (split < tile * tiles)
+            {
+                a.part = (float*)prefill_scratch_try(bytes, stream, 4);
+                if (a.part) a.splits = n;
+            }
         }
+        if (getenv("EXL2_DEBUG_ROUTE")) fprintf(stderr, "flash_prefill route: key splits=%d\n", a.splits);
     }
     dim3 grid((unsigned)((q_len + FP_BQ - 1) / FP_BQ), (unsigned)num_heads, (unsigned)(batch * a.splits));
     const size_t lds = ((size_t)FP_BK * (head_dim + 8) + (size_t)FP_BK * (head_dim + 16)) * sizeof(f16);

@@ -390,6 +390,19 @@ def test_flash_prefill_key_splits(be, hd, nh, kvh, s, past, causal):
     assert np.all(np.abs(got - want.astype(np.float32)) <= _attn_tol(want.astype(np.float32))), float(np.abs(got - want).max())
 
 
+@pytest.mark.parametrize("s,past,splits", [(37, 600, 5), (333, 0, 1), (200, 100, 1), (200, 600, 6)])
+def test_flash_prefill_key_splits_where_they_pay(be, s, past, splits, capfd, monkeypatch):
+    """32 heads: few rows behind many keys are split, the start of a prompt, whose partial results alone cost more than its tiles, is not."""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    rng = np.random.default_rng(s)
+    q, k, v = (rng.standard_normal((1, n, h, 64)).astype(F16) for n, h in ((s, 32), (past + s, 2), (past + s, 2)))
+    out = torch.zeros((1, s, 32, 64), dtype=torch.float16, device=be.device)
+    assert be.ext.flash_prefill(be.t(q), be.t(k), be.t(v), out, None, None, len_const=past, len_offset=s)
+    assert f"flash_prefill route: key splits={splits}\n" in capfd.readouterr().err
+    want = OM.attention(q, k, v).astype(np.float32)
+    assert np.all(np.abs(be.n(out).astype(np.float32) - want) <= _attn_tol(want))
+
+
 @pytest.mark.parametrize("s, past", [(200, 400), (20, 900)])
 def test_flash_prefill_nan_scores(be, s, past):
     """A key whose scores are NaN counts as no key, in the tiles that need no mask as in the others, with key splits and without."""
