@@ -423,7 +423,7 @@ int exl2_flash_prefill_ex(const void* q, const void* k_cache, const void* v_cach
     // 1.3 of it with two workgroups) against the merging launch (2 us, 0.5 per split, 0.45 per MB of partial results).
     // Whole calls on the MI355X, us, in one split | in the rule's number: 32 heads of 128, 37 rows behind 600 keys 25.3 | 13.8 in five, 200
     // behind 600 32.2 | 22.7 in six, 333 behind 2000 83.1 | 42.3 in five; 64 heads, 37 behind 8000 267 | 59.6 in eight.  Where it does not:
-    // 333 rows of a prompt's start 17.0 (three splits: 23.1), 500 rows 22.3 (four: 25.6).  Of 310 shapes (8 - 64 heads of 64, 128, 256, 4 -
+    // 333 rows of a prompt's start 17.0 (three splits: 23.1), 500 rows 22.3 (four: 25.6).  Of 297 shapes (8 - 64 heads of 64, 128, 256, 4 -
     // 1024 rows behind 0 - 8000 keys) none that it splits is slower for it, one that it leaves (31.5) would gain 1.8
     a.splits = 1;
     if (!ws && !cache_seqlens)

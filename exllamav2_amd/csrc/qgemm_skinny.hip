@@ -529,12 +529,15 @@ int qgemm_skinny_launch(const PrefillArgs* pas, int n, bool gptq, void* stream)
     for (int i = n + 1; i <= SK_MAX_JOBS; i++) p.group0[i] = 0x7fffffff;
     const size_t lds = gptq ? (size_t)SK_LDS_BYTES(RBT, 1, K >> 5) : (size_t)SK_LDS_BYTES(RBT, 0, K >> 5);
     if (lds > 160 * 1024) return 1;
-    // K splits: as many as fit the chip in one round, 8 at most, >= 2 items per split.  Whole calls, us (rows: 1 .. 16 splits): 4096 x 4096 at
-    // 48 rows 2: 26.5, 4: 21.5, 8: 19.4, 16: 24.7; 11008 x 4096 2: 54.9, 4: 38, 8: 32.6, 16: 34.3; 4096 x 22016 2: 33.6, 4: 33.1, 8: 43.6
-    // (two rounds).  More splits are more bytes for the adding launch.
+    // K splits: as many as fit the chip in one round (two workgroups per CU up to 32 rows, whatever fits from 33), 8 at most; >= 4 items per
+    // split beyond four of them.  Whole calls over weights that come from memory, us (splits: time).  48 rows: 4096 x 4096 2: 24.9, 4: 19.6,
+    // 8: 18.8; 11008 x 4096 2: 51.4, 4: 35.7, 8: 29.2; 4096 x 22016 2: 34.4, 4: 33.5, 8: 43.5 (two rounds); 2048 x 5632 2: 17.9, 4: 16.2, 8: 19.7
+    // (two items each).  17 rows: 4096 x 11008 2: 23.3, 4: 21.2, 5: 22.6, 8: 23.2; 4096 x 32000 1: 34.7, 2: 33.0, 3: 34.9; 8192 x 28672 (8 / 4 bits)
+    // 2: 55.7, 3: 57.1.  More splits are more bytes for the adding launch.
     const int per_cu = (int)((160 * 1024) / lds) < (RBT <= 4 ? 3 : 2) ? (int)((160 * 1024) / lds) : (RBT <= 4 ? 3 : 2);
-    int ks = 256 * per_cu / groups;
+    int ks = 256 * (RBT <= 2 ? 2 : per_cu) / groups;
     if (ks > 8) ks = 8;
+    if (ks > 4 && ks > min_items / 4) ks = min_items / 4 > 4 ? min_items / 4 : 4;
     if (ks > min_items / 2) ks = min_items / 2;
     if (const char* e = getenv("EXL2_SKINNY_SPLITK")) { const int v = atoi(e); if (v >= 1) ks = v > 32 ? 32 : v; if (ks > min_items) ks = min_items; }
     if (ks < 1) ks = 1;

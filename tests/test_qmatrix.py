@@ -214,6 +214,20 @@ def test_prefill_tile256_variant_forced(be, m, wpre, mt, monkeypatch):
     be.ext.free_q_matrix(h)
 
 
+@pytest.mark.parametrize("k,n,m,ks", [(1024, 256, 17, 4), (1024, 32, 64, 4), (2048, 64, 32, 4), (2048, 64, 33, 4), (4096, 32, 17, 8), (2560, 32, 32, 5)])
+def test_skinny_split_counts(be, k, n, m, ks, capfd, monkeypatch):
+    """How many K splits 17 - 64 rows take where the columns leave CUs idle: at least four items each beyond four splits."""
+    monkeypatch.setenv("EXL2_SKINNY_DEBUG", "1")
+    t, ref, w, h = make_exl2(be, k, n, [(4, 128, k)], seed=61)
+    a = np.random.default_rng(62).standard_normal((m, k)).astype(np.float16)
+    c = torch.zeros((m, n), dtype=torch.float16, device=be.device)
+    be.ext.gemm_half_q_half(be.t(a), h, c)
+    assert f" grid {(n + 127) // 128} x {ks} " in capfd.readouterr().err
+    want = OX.gemm_ref(a, ref, exact=True)
+    assert np.all(np.abs(be.n(c).astype(np.float64) - want) <= half_tol(want, k))
+    be.ext.free_q_matrix(h)
+
+
 @pytest.mark.parametrize("name", ["b3", "mixed_all", "long_runs"])
 @pytest.mark.parametrize("m,ks", [(33, 1), (48, 2), (65, 4), (96, 3), (97, 2)])
 def test_skinny_row_blocks(be, name, m, ks, monkeypatch):
