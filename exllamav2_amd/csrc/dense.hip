@@ -143,7 +143,7 @@ DEV void lin_rows_fma(const u32x4 (&wq)[C], const u32x4 (&xq)[MB], float (&acc)[
 // run in K order whatever C and U are.  bf16, us (read at the rate of a large copy | one column, a step at a time | now), K x N at 1 / 4 / 16 rows:
 //   2048 x 8512:  7.2 | 11.3 / 14.5 / 35.3 | 8.5 / 11.4 / 19.6      8192 x 2048: 6.9 | 13.3 / 16.0 / 29.5 | 9.1 / 11.0 / 20.5
 //   2048 x 32000: 27  | 28.1 / 39.4 / 118  | 24.4 / 31.8 / 63.7     2048 x 2048: 1.7 | 5.4 / 7.2 / 11.5   | 4.5 / 5.5 / 7.8
-// (four columns: 12.8, 15.0, 30.3, 6.9 at 4 rows)
+// (four columns: 12.8, 15.0, 30.3, 6.9 at 4 rows; where one column is kept: launch_rows_mb)
 template <typename T, typename TY, int MB, bool VEC, int C>
 KERNEL void __launch_bounds__(256) lin_rows_kernel(const LinArgs a)
 {
@@ -496,11 +496,26 @@ KERNEL void __launch_bounds__(256) lin_mfma_tile_kernel(const LinArgs a)
 
 // ---- host -------------------------------------------------------------------------------------------------------------------
 
+template <typename T, typename TY, int MB, bool VEC, int C>
+static void launch_rows_c(const LinArgs& a, int batch, hipStream_t s)
+{
+    LAUNCH((lin_rows_kernel<T, TY, MB, VEC, C>), dim3((a.N + 4 * C - 1) / (4 * C), a.w_sel ? a.M : (a.M + MB - 1) / MB, batch), dim3(256), 0, s, a);
+}
+
+// Two columns per wave where one leaves no CU without a workgroup: below that a wave's own chain is the time, and two columns make it longer.
+// fp32 rows, twice the bytes, need several workgroups per CU up to four rows.  One | two columns, us, weights from memory, K = 8192: bf16 2 / 4 /
+// 16 rows N = 1024 6.9 | 7.9, 8.5 | 10.0, 17.0 | 14.5; N = 4096 16.2 | 15.9, 23.0 | 18.6, 54.9 | 36.4; fp32 N = 1024 9.8 | 13.8, 15.3 | 20.6,
+// 27.1 | 23.3; N = 4096 29.3 | 32.9, 42.9 | 36.1, 107 | 65; N = 64 5 rows 21.3 | 19.8
 template <typename T, typename TY, int MB, bool VEC>
 static void launch_rows_mb(const LinArgs& a, int batch, hipStream_t s)
 {
-    constexpr int C = VEC && MB > 1 ? 2 : 1;
-    LAUNCH((lin_rows_kernel<T, TY, MB, VEC, C>), dim3((a.N + 4 * C - 1) / (4 * C), a.w_sel ? a.M : (a.M + MB - 1) / MB, batch), dim3(256), 0, s, a);
+    if constexpr (VEC && MB > 1)
+    {
+        const long long wgs = (long long)((a.N + 3) / 4) * ((a.M + MB - 1) / MB) * batch;
+        const int per_cu = sizeof(T) == 2 ? 1 : MB == 2 ? 4 : MB == 4 ? 2 : 0;
+        if (wgs > 256LL * per_cu) { launch_rows_c<T, TY, MB, VEC, 2>(a, batch, s); return; }
+    }
+    launch_rows_c<T, TY, MB, VEC, 1>(a, batch, s);
 }
 
 template <typename T, typename TY, bool VEC>

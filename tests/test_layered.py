@@ -63,10 +63,11 @@ def test_dense_linear(be, dtype, M, N, K, epi):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
-@pytest.mark.parametrize("M,N,K", [(1, 5, 2048), (2, 9, 2568), (3, 1, 4096), (4, 17, 1032), (5, 8, 1024), (8, 7, 3080), (9, 9, 2048), (16, 16, 520)])
+@pytest.mark.parametrize("M,N,K", [(1, 5, 2048), (2, 9, 2568), (3, 1, 4096), (4, 17, 1032), (5, 8, 1024), (8, 7, 3080), (9, 9, 2048), (16, 16, 520),
+                                   (2, 1024, 520), (2, 1025, 520), (4, 1027, 1032), (4, 2049, 264), (2, 4097, 264), (9, 515, 1032), (16, 513, 520)])
 def test_dense_linear_columns_in_pairs(be, dtype, M, N, K):
-    """A wave's two columns and its several K steps in flight (csrc/dense.hip: lin_rows_kernel): an odd last column, K with whole passes, left
-    steps and a step that not all lanes have.  A lane sums K / 64 products (+ the steps rounded up), then six additions over the lanes."""
+    """A wave's one or two columns and its several K steps in flight (csrc/dense.hip: lin_rows_kernel), on both sides of the line between one
+    and two: an odd last column, K with whole passes, left steps and a step that not all lanes have.  A lane sums K / 64 products (+ the steps rounded up), then six additions over the lanes."""
     rng = np.random.default_rng(M * 1000 + N * 10 + K)
     x, w = bf16_exact(rng.standard_normal((M, K))).astype(np.float64), bf16_exact(rng.standard_normal((N, K)) / math.sqrt(K)).astype(np.float64)
     aux = rng.standard_normal((M, N)).astype(np.float32)
