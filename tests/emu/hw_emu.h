@@ -468,7 +468,8 @@ DEV hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = aligned_alloc(
 // graphs cannot be emulated: capture is refused, callers fall back to eager launches in the emu tests
 typedef void* hipGraph_t;
 enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1 };
-DEV hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) { *s = hipStreamCaptureStatusNone; return hipSuccess; }
+// (EXL2_EMU_CAPTURING: what a launch sees inside a capture -- scratch that cannot grow)
+DEV hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) { *s = getenv("EXL2_EMU_CAPTURING") ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone; return hipSuccess; }
 typedef void* hipGraphExec_t;
 enum { hipStreamCaptureModeRelaxed = 2 };
 DEV hipError_t hipStreamBeginCapture(hipStream_t, int) { return hipErrorInvalidValue; }

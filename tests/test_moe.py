@@ -30,23 +30,36 @@ def test_moe_route(be, experts, topk):
     assert np.allclose(got.astype(np.float32).sum(-1), 1.0, atol=2e-3)
 
 
-def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31, spec_up=None, spec_dn=None, gate_scale=0.3, spec_w3=None, max_rows=128, bias=0.0):
+def _gelu_mul(gate, up):
+    """the tanh form of GELU in float32, rounded to fp16, times up (cuda/q_mlp_activation.cuh's order)"""
+    g = gate.astype(np.float64)
+    y = (0.5 * g * (1.0 + np.tanh(0.797884560803 * (g + 0.044715 * g ** 3)))).astype(F16)
+    return np.clip(OM.hmul(y, up), F16(-65504.0), F16(65504.0))
+
+
+def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31, spec_up=None, spec_dn=None, gate_scale=0.3, spec_w3=None, max_rows=128, bias=0.0, gptq=0, gelu=False, run=None):
     """one sparse-MoE block (q_moe_mlp_forward_) against the oracle's composition: routing mask, weighted expert sum into the residual.
-    bias: root mean square of the biases of down (gate and up: a quarter of it), none at 0"""
-    from tests.util import exl2_to_torch
+    bias: root mean square of the biases of down (gate and up: a quarter of it), none at 0.
+    gptq: the experts' group size, 0 = EXL2; run(moe, x): what runs the block in the place of q_moe_mlp_forward_"""
+    from tests.util import exl2_to_torch, gptq_to_torch
     rng = np.random.default_rng(seed)
     spec_up = spec_up or [(5, 32, 32), (4, 32, hidden - 32)]
     spec_dn = spec_dn or [(5, 32, 64), (4, 64, inter - 64)]
     keep, handles, refs, biases = [], {"w1": [], "w2": [], "w3": []}, {"w1": [], "w2": [], "w3": []}, {"w1": [], "w2": [], "w3": []}
     shared = rng.permutation(hidden).astype(np.int32)
+    shared_g = rng.permutation(np.arange(hidden) // gptq).astype(np.int32) if gptq else None
     for e in range(E):
         for name, (k, n, spec) in (("w1", (hidden, inter, spec_up)), ("w3", (hidden, inter, spec_w3 or spec_up)), ("w2", (inter, hidden, spec_dn))):
-            t = OX.synth_exl2(k, n, spec, seed=100 + 3 * e + len(name) + ord(name[1]), act_order=True)
+            if gptq:
+                t = OX.synth_gptq(k, n, gptq, seed=100 + 3 * e + ord(name[1]), act_order=True)
+                t["scales"] = (t["scales"] * F16(0.5)).astype(F16)
+                if shared_perm and name != "w2": t["g_idx"] = shared_g.copy()
+            else: t = OX.synth_exl2(k, n, spec, seed=100 + 3 * e + len(name) + ord(name[1]), act_order=True)
             if bias: t["bias"] = (np.random.default_rng([seed, e, k, n]).standard_normal(n) * (bias if name == "w2" else bias / 4)).astype(F16)
-            if shared_perm and name != "w2":
+            if shared_perm and name != "w2" and not gptq:
                 t["q_invperm"] = shared.copy()
-            ref = OX.exl2_reconstruct(t)
-            w = exl2_to_torch(be, t)
+            ref = OX.gptq_reconstruct(t) if gptq else OX.exl2_reconstruct(t)
+            w = gptq_to_torch(be, t) if gptq else exl2_to_torch(be, t)
             h = be.ext.make_q_matrix_from_dict(w, None)
             keep.append(w); handles[name].append(h); refs[name].append(ref); biases[name].append(t.get("bias"))
     norm_w = (1.0 + 0.1 * rng.standard_normal(hidden)).astype(F16)
@@ -62,9 +75,10 @@ def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31
     from exllamav2_amd.ext import none_tensor
     nw, gt = be.t(norm_w), be.t(gate)
     moe = be.ext.make_q_moe_mlp(nw, none_tensor, True, 1e-5, gt, E, topk, handles["w1"], handles["w2"], handles["w3"],
-                                ts, none_tensor, ta, tb, tl, none_tensor, max_rows, False)
+                                ts, none_tensor, ta, tb, tl, none_tensor, max_rows, gelu)
     xt = be.t(x)
-    be.ext.q_moe_mlp_forward_(moe, xt)
+    if run: run(moe, xt)
+    else: be.ext.q_moe_mlp_forward_(moe, xt)
     got = be.n(xt).astype(np.float64)
 
     # oracle composition
@@ -86,7 +100,7 @@ def _moe_case(be, rows, shared_perm, E=8, topk=2, hidden=128, inter=256, seed=31
         if len(sel) == 0: continue
         g = OX.gemm_ref(xn[sel], refs["w1"][e], bias=biases["w1"][e], exact=True).astype(F16)
         u = OX.gemm_ref(xn[sel], refs["w3"][e], bias=biases["w3"][e], exact=True).astype(F16)
-        a = OM.silu_mul(g, u)
+        a = _gelu_mul(g, u) if gelu else OM.silu_mul(g, u)
         d = OX.gemm_ref(a, refs["w2"][e], bias=biases["w2"][e], exact=True)
         want[sel] += d * wts[sel, e].astype(np.float64)[:, None]
     tol = np.abs(want) * 2.0 ** -8 + 6e-3                   # E sequential fp16 accumulations into the residual
@@ -165,6 +179,68 @@ def test_moe_experts_with_biases_launch_by_launch(be, rows, shared_perm, env, mo
     the product."""
     if env: monkeypatch.setenv(env, "1")
     _moe_case(be, rows, shared_perm, gate_scale=0.6, bias=2.0)
+
+
+@pytest.mark.parametrize("gptq,gelu", [(32, False), (32, True), (0, True)])
+@pytest.mark.parametrize("rows,tile_rb,route", [(2, None, "slots"), (17, None, "slots"), (33, None, "slots"), (64, None, "slots"), (70, 2, "tiles"), (70, 4, "tiles"), (130, 8, "tiles")])
+def test_moe_gptq_and_gelu_experts(be, rows, tile_rb, route, gptq, gelu, capfd, monkeypatch):
+    """GPTQ experts (zero points beside the scales) and GELU units in the kernels that run all experts in one launch, at every number of row blocks"""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    if tile_rb: monkeypatch.setenv("EXL2_TILE_RB", str(tile_rb))
+    _moe_case(be, rows, True, E=4, hidden=128, inter=288, gate_scale=0.6, max_rows=160, gptq=gptq, gelu=gelu, bias=0.5, spec_dn=[(5, 32, 64), (3, 32, 224)])
+    assert f"route: {route}" in capfd.readouterr().err
+
+
+@pytest.mark.parametrize("gptq", [0, 32])
+def test_moe_tiles_without_a_pair(be, gptq, capfd, monkeypatch):
+    """17 rows on: experts whose gate and up are cut into different sections (GPTQ: always alike, a pair)"""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    for rows in (17, 33, 64):
+        _moe_case(be, rows, True, gate_scale=0.6, spec_w3=[(6, 32, 64), (4, 32, 64)], max_rows=160, bias=0.5, gptq=gptq)
+        err = capfd.readouterr().err
+        assert ("route: slots" in err) if gptq else ("route: tiles" in err and "pair" not in err)
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("rows,hidden", [(2, 128), (5, 2176), (16, 160)])
+def test_moe_slots_publish_for_the_next_consumer(be, rows, hidden, tiled, capfd, monkeypatch):
+    """The slots route inside a chained step: its last launch leaves x times the next consumer's norm weight in that consumer's order (plain and
+    tiled) and the partial sums of squares of every row, one per workgroup."""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    rng = np.random.default_rng(71)
+    inv = rng.permutation(hidden).astype(np.uint16)
+    norm = (1.0 + 0.2 * rng.standard_normal(hidden)).astype(F16)
+    invt, normt = be.t(inv.view(np.int16)), be.t(norm)
+    xp = torch.zeros((16 * hidden,), dtype=torch.float16, device=be.device)
+    ss = torch.zeros((rows, 512), dtype=torch.float32, device=be.device)
+    seen = {}
+
+    def run(moe, xt):
+        be.ext.chain_set_tiled(tiled)
+        try: seen["n"] = be.ext.q_moe_mlp_forward_chain(moe, xt, rows, invt.data_ptr(), normt, xp, ss)
+        finally: be.ext.chain_set_tiled(False)
+        seen["x"] = be.n(xt).copy()
+
+    _moe_case(be, rows, True, E=4, hidden=hidden, inter=160, gate_scale=0.6, run=run)
+    assert "route: slots" in capfd.readouterr().err and seen["n"] == (hidden // 8 + 255) // 256
+    x = seen["x"].astype(np.float32)
+    want = np.zeros((rows, hidden), dtype=F16)
+    want[:, inv.astype(np.int64)] = (x * norm.astype(np.float32)[inv.astype(np.int64)]).astype(F16)
+    got = be.n(xp)
+    got = got.reshape(hidden // 8, 16, 8).transpose(1, 0, 2).reshape(16, hidden)[:rows] if tiled else got.reshape(16, hidden)[:rows]
+    assert np.array_equal(got.view(np.uint16), want.view(np.uint16))
+    sums = be.n(ss).reshape(-1)[:rows * seen["n"]].reshape(rows, seen["n"]).sum(-1)
+    # (fp32: 8 terms per lane, then 6 + 2 additions)
+    assert np.all(np.abs(sums - (x.astype(np.float64) ** 2).sum(-1)) <= 20 * 2.0 ** -24 * (x.astype(np.float64) ** 2).sum(-1))
+
+
+@pytest.mark.parametrize("be", ["emu"], indirect=True)
+@pytest.mark.parametrize("rows", [2, 17, 64, 80])
+def test_moe_without_scratch(be, rows, monkeypatch):
+    """Scratch that cannot be had (as inside a capture on a stream that holds none): the routes that need none answer."""
+    be.ext.release_scratch()
+    monkeypatch.setenv("EXL2_EMU_CAPTURING", "1")
+    _moe_case(be, rows, True, gate_scale=0.6, bias=0.5)
 
 
 def test_moe_model_forward(be):

@@ -289,6 +289,31 @@ def test_prefill_matrices_over_the_same_rows_share_a_launch(be, monkeypatch):
     assert outs[3] - outs[1] == 3 * cfg.num_hidden_layers
 
 
+@pytest.mark.parametrize("be", ["emu"], indirect=True)
+@pytest.mark.parametrize("m,ks_env,pre_env", [(48, "EXL2_SKINNY_SPLITK", None), (130, "EXL2_PREFILL_KS", None), (130, "EXL2_PREFILL_KS", "EXL2_PREFILL_WPRE_MIN_ROWS")])
+def test_splits_and_fragments_without_scratch(be, m, ks_env, pre_env, capfd, monkeypatch):
+    """Scratch for the staged rows but none for partial tiles or weight fragments (as inside a capture): one split, decode in the product."""
+    k, n, spec = SPECS["mixed_all"]
+    t, ref, w, h = make_exl2(be, k, n, spec, seed=55, bias=True)
+    a = np.random.default_rng(56).standard_normal((m, k)).astype(np.float16)
+    c = torch.zeros((m, n), dtype=torch.float16, device=be.device)
+    be.ext.release_scratch()
+    monkeypatch.setenv(ks_env, "1")
+    monkeypatch.setenv("EXL2_PREFILL_WPRE_MIN_ROWS", "0")
+    be.ext.gemm_half_q_half(be.t(a), h, c)
+    c.zero_()
+    monkeypatch.setenv(ks_env, "2")
+    if pre_env: monkeypatch.setenv(pre_env, "1")
+    monkeypatch.setenv("EXL2_EMU_CAPTURING", "1")
+    monkeypatch.setenv("EXL2_SKINNY_DEBUG", "1"); monkeypatch.setenv("EXL2_PREFILL_TRACE", "1")
+    be.ext.gemm_half_q_half(be.t(a), h, c)
+    err = capfd.readouterr().err
+    assert (" x 1 lds" in err) if m <= 128 else ("splits=1 " in err and "pre=0" in err)
+    want = OX.gemm_ref(a, ref, bias=t["bias"], exact=True)
+    assert np.all(np.abs(be.n(c).astype(np.float64) - want) <= half_tol(want, k))
+    be.ext.free_q_matrix(h)
+
+
 def test_prefill_matrix_of_many_sections_beside_one_of_few(be, capfd, monkeypatch):
     """gate in one section, up in more than a kernel's argument block names: up decodes inside its product, gate's weights are decoded ahead as
     they are alone -- the two do not share a launch."""
