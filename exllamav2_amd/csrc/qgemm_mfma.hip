@@ -387,39 +387,6 @@ KERNEL void __launch_bounds__(MF_THREADS) wfrag_kernel(const MfArgs args)
     }
 }
 
-// four consecutive columns n .. n + 3 of one row of the result: bias, accumulate-into-c, the consumer's column order
-DEV void mf_store(const MfJob& job, int row, int n, f32x4 v)
-{
-    f16* const cp = job.c + (size_t)row * job.ldc;
-    if (job.m.bias)
-    {
-        #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] += (float)job.m.bias[n + e];
-    }
-    if (!job.c_invperm && !(job.ldc & 3) && !(((size_t)job.c) & 7))
-    {
-        f16x4 h;
-        if (job.c_mode == C_ACCUM)
-        {
-            const f16x4 old = *(const f16x4*)(cp + n);
-            #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] += (float)old[e];
-        }
-        #pragma unroll
-        for (int e = 0; e < 4; e++) h[e] = (f16)v[e];
-        *(f16x4*)(cp + n) = h;
-        return;
-    }
-    #pragma unroll
-    for (int e = 0; e < 4; e++)
-    {
-        const int nn = job.c_invperm ? (int)job.c_invperm[n + e] : n + e;
-        float w = v[e];
-        if (job.c_mode == C_ACCUM) w += (float)cp[nn];
-        cp[nn] = (f16)w;
-    }
-}
-
 template <bool GPTQ, int MT, bool WPRE>
 KERNEL void __launch_bounds__(MF_THREADS, 2) qgemm_mfma_kernel(const MfArgs args)
 {
@@ -552,7 +519,7 @@ KERNEL void __launch_bounds__(MF_THREADS, 2) qgemm_mfma_kernel(const MfArgs args
         for (int mt = 0; mt < MT; mt++)
         {
             const int row = m0 + wm * MT * 16 + mt * 16 + i16;
-            if (row < M) mf_store(job, row, n, acc[mt][nt]);
+            if (row < M) store_row4(job, row, n, acc[mt][nt]);
         }
     }
 }
@@ -575,7 +542,7 @@ KERNEL void __launch_bounds__(256) mf_reduce_kernel(const MfArgs args)
     const f32x4* p = args.part + (size_t)tn * args.ks * PER + u;
     f32x4 acc = p[0];
     for (int z = 1; z < args.ks; z++) acc += p[(size_t)z * PER];
-    mf_store(job, row, n, acc);
+    store_row4(job, row, n, acc);
 }
 
 // ---- host ---------------------------------------------------------------------------------------------------------------

@@ -25,3 +25,37 @@ int qgemm_skinny_launch(const PrefillArgs* p, int n, bool gptq, void* stream);  
 
 // qgemm_mfma.hip: 0 = launched, < 0 = error (message set)
 int qgemm_mfma_launch(const PrefillArgs* p, int n, bool gptq, void* stream);       // n <= 3 matrices over the same staged rows
+
+// four consecutive columns n .. n + 3 of one row of the result: bias, accumulate-into-c, the consumer's column order (JOB: m, c,
+// c_invperm, ldc, c_mode)
+template <typename JOB> DEV void store_row4(const JOB& job, int row, int n, f32x4 v)
+{
+    f16* const cp = job.c + (size_t)row * job.ldc;
+    if (job.m.bias)
+    {
+        #pragma unroll
+        for (int e = 0; e < 4; e++) v[e] += (float)job.m.bias[n + e];
+    }
+    if (!job.c_invperm && !(job.ldc & 3) && !(((size_t)job.c) & 7))
+    {
+        f16x4 h;
+        if (job.c_mode == C_ACCUM)
+        {
+            const f16x4 old = *(const f16x4*)(cp + n);
+            #pragma unroll
+            for (int e = 0; e < 4; e++) v[e] += (float)old[e];
+        }
+        #pragma unroll
+        for (int e = 0; e < 4; e++) h[e] = (f16)v[e];
+        *(f16x4*)(cp + n) = h;
+        return;
+    }
+    #pragma unroll
+    for (int e = 0; e < 4; e++)
+    {
+        const int nn = job.c_invperm ? (int)job.c_invperm[n + e] : n + e;
+        float w = v[e];
+        if (job.c_mode == C_ACCUM) w += (float)cp[nn];
+        cp[nn] = (f16)w;
+    }
+}

@@ -202,38 +202,6 @@ DEV SkSegment sk_segment(const QMatDev& m, int i)
     return g;
 }
 
-// four consecutive columns n .. n + 3 of one row of the result: bias, accumulate-into-c, the consumer's column order
-DEV void sk_store(const SkinnyJob& job, int row, int n, f32x4 v)
-{
-    f16* const cp = job.c + (size_t)row * job.ldc;
-    if (job.m.bias)
-    {
-        #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] += (float)job.m.bias[n + e];
-    }
-    if (!job.c_invperm && !(job.ldc & 3) && !(((size_t)job.c) & 7))
-    {
-        f16x4 h;
-        if (job.c_mode == C_ACCUM)
-        {
-            const f16x4 old = *(const f16x4*)(cp + n);
-            #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] += (float)old[e];
-        }
-        #pragma unroll
-        for (int e = 0; e < 4; e++) h[e] = (f16)v[e];
-        *(f16x4*)(cp + n) = h;
-        return;
-    }
-    #pragma unroll
-    for (int e = 0; e < 4; e++)
-    {
-        const int nn = job.c_invperm ? (int)job.c_invperm[n + e] : n + e;
-        float w = v[e];
-        if (job.c_mode == C_ACCUM) w += (float)cp[nn];
-        cp[nn] = (f16)w;
-    }
-}
 DEV int sk_job(const SkinnyArgs& a, int group) { return (group >= a.group0[1] ? 1 : 0) + (group >= a.group0[2] ? 1 : 0); }
 
 template <bool GPTQ, int RB>
@@ -318,7 +286,7 @@ KERNEL void __launch_bounds__(SK_THREADS, RB <= 4 ? 3 : 2) qgemm_skinny_kernel(c
         for (int rb = 0; rb < RB; rb++)
         {
             const int row = rb * 16 + (lane & 15);
-            if (row < args.M) sk_store(job, row, n, acc[rb][ct]);
+            if (row < args.M) store_row4(job, row, n, acc[rb][ct]);
         }
     }
 }
@@ -337,7 +305,7 @@ KERNEL void __launch_bounds__(256) sk_reduce_kernel(const SkinnyArgs args)
     const f32x4* p = args.part + (size_t)grp * args.ks * PER + u;
     f32x4 acc = p[0];
     for (int z = 1; z < args.ks; z++) acc += p[(size_t)z * PER];
-    sk_store(job, row, n, acc);
+    store_row4(job, row, n, acc);
 }
 
 // ---- experts of a sparse block, 2 .. 64 rows (qgemm_skinny.h) ------------------------------------------------------------------------
