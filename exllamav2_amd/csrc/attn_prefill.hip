@@ -210,7 +210,8 @@ KERNEL void __launch_bounds__(FP_WAVES * 64, FP_OCC) flash_prefill_kernel(const 
         // sees whole (all but the last one or two of a causal block) needs no mask: per score one maximum, one fused multiply-add into
         // the exponent, the exponential and the sum.  (A NaN score shows in the sum.  The fused exponent of the largest key is the rounding of the
         // maximum and not 0: it scales the row's probabilities alike, by 1/e to e up to 2^24.  Tiles beyond either go the general way.)
-        // Causal 8 x 2048 rows of 32 heads of 128: 755 us with the mask and the rescale in every tile, 685 so (0.40 PFLOP/s over the visible scores).
+        // Causal 8 x 2048 rows of 32 heads of 128, back to back by itself: 755 us with the mask and the rescale in every tile, 692 so (0.40 PFLOP/s
+        // over the visible scores); 766 between the products of a model's layer, where the chip is at its power limit.
         f16x8 pb[RPW][NBLK / 2];                     // B operands: 32 keys each = {block 2n keys 4g..4g+3, block 2n+1 keys 4g..4g+3}
         float alpha[RPW];
         const bool whole = !WS && a.scale > 0.0f && k0 + FP_BK <= total && (!a.causal || k0 + FP_BK - 1 <= qpos0 + q0 + wv * RPW * 16);

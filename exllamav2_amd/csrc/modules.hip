@@ -138,7 +138,7 @@ struct QMoEMLP
     // kernel of a step copies the selected ones to the slots the gate|up and the down launch read (qgemv_lean.h: LeanGroupPlan)
     bool lean_ok; LeanGroupPlan lean_gu, lean_dn;
     bool lean_rows_ok[LEAN_MAX_M + 1]; LeanGroupPlan lean_gu_r[LEAN_MAX_M + 1], lean_dn_r[LEAN_MAX_M + 1];      // 2-4 rows: one launch over all experts each (the reference's fused form covers <= 4 rows, q_mlp.cu:316-436)
-    // more than 16 rows: all experts in one launch per projection (qgemm_tile.hip); device tables made here
+    // 2 rows on: all experts in one launch per projection (qgemm_skinny.hip, qgemm_tile.hip); device tables made here
     bool tile_ok, tile_pair; QMatDev* tile_mats; const u16** tile_invperms;      // [E][w1, w3, w2]; [E] w2's packed order (null: natural order)
     bool down_bias;                             // some expert's w2 has a bias
     bool lean_sum_ok; LeanGroupPlan lean_dn2;      // top-2: both selected experts' down projections as ONE pair launch that adds the weighted sum to x (no combine launch)
@@ -709,8 +709,8 @@ int exl2_free_q_moe_mlp(void* handle)
 // q_moe_mlp_forward_ (ext_qmlp.cpp:245-272 -> QMoEMLP::forward_, q_mlp.cu:318-402): in place on x [rows, hidden].
 // The reference takes rows <= 4; here any row count.  One row: the lean kernels over the chosen experts.  2 .. 64: moe_forward_slots, all
 // experts over the rows that chose them.  More: moe_forward_tile, over lists of them (1093 rows of a 4096 x 14336 x 8 block: 1.15 ms, in
-// passes of 16 rows 43 ms).  Experts that share no packed order, or whose gate and up are cut into different sections (2 .. 64 rows):
-// the routes below, 16 rows at a time.
+// passes of 16 rows 43 ms).  Experts whose gate and up are cut into different sections: the grouped launches up to 16 rows, moe_forward_tile
+// from 17 on.  Experts that share no packed order, or scratch that cannot be had: the routes at the end, 16 rows at a time.
 static int moe_forward(void* handle, void* x_, int rows, const MoeChainOut& co, int* npart_out, void* stream)
 {
     EXL2_REQUIRE(handle && x_, "q_moe_mlp_forward_: null argument");
@@ -806,8 +806,8 @@ static int moe_forward(void* handle, void* x_, int rows, const MoeChainOut& co, 
         const int rc = moe_forward_slots(m, x, have_xg ? xg : nullptr, rows, co, npart_out, stream);
         if (rc <= 0) return rc;
     }
-    // ---- (gate and up cut into different sections) grouped route (rows <= 16): all experts' gate|up in ONE launch (SiLU * up in the epilogue, written in each down
-    // projection's packed order), all experts' down in ONE launch (weighted partial outputs), one combine.  Replaces the
+    // ---- gate and up cut into different sections: grouped route (rows <= 16): all experts' gate|up in ONE launch (SiLU * up in the epilogue,
+    // written in each down projection's packed order), all experts' down in ONE launch (weighted partial outputs), one combine.  Replaces the
     // per-expert launch loop below (3 launches per expert: q_mlp.cu:318-402 has the same shape, moe_mlp.py:255-323 a
     // Python loop above 4 rows).
     if (m->group_ok && rows <= MAX_GEMV_ROWS && 2 * MAX_GEMV_ROWS <= m->max_rows && (long long)E * rows <= m->max_rows &&

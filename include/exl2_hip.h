@@ -249,7 +249,7 @@ int exl2_q_mlp_forward(void* handle, void* x, int rows, void* stream);
 
 /* make_q_moe_mlp / q_moe_mlp_forward_ (ext_qmlp.h, ext_qmlp.cpp:245-272 -> QMoEMLP::forward_ cuda/q_mlp.cu:318-402).
    w1 / w2 / w3: arrays of num_experts q_matrix handles (gate, down, up projections).  num_experts in {4, 8, 16}.
-   The reference accepts rows <= 4; this entry point takes any rows <= max_rows (16-row passes). */
+   The reference accepts rows <= 4; this entry point takes any rows <= max_rows. */
 int exl2_make_q_moe_mlp(void** handle, const void* layernorm, const void* layernorm_bias, int layernorm_is_rms,
                         float norm_epsilon, const void* gate, int num_experts, int num_experts_per_token,
                         void* const* w1, void* const* w2, void* const* w3, void* temp_state, void* temp_gathered_state,

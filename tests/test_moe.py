@@ -144,7 +144,8 @@ def test_moe_many_rows_all_experts_in_one_launch(be, rows, E, topk, hidden, inte
     assert "route: tiles" in err and "pair" not in err
 
 
-@pytest.mark.parametrize("rows,E,topk,hidden,inter,ks", [(2, 8, 2, 128, 160, 2), (5, 8, 2, 128, 256, 1), (16, 4, 2, 160, 224, 2), (17, 8, 2, 128, 160, 3), (32, 4, 3, 256, 288, 2), (33, 16, 1, 128, 128, 1), (64, 4, 2, 128, 224, 3)])
+@pytest.mark.parametrize("rows,E,topk,hidden,inter,ks", [(2, 8, 2, 128, 160, 2), (5, 8, 2, 128, 256, 1), (16, 4, 2, 160, 224, 2), (17, 8, 2, 128, 160, 3), (32, 4, 3, 256, 288, 2), (33, 16, 1, 128, 128, 1), (64, 4, 2, 128, 224, 3),
+                                                        (9, 8, 2, 128, 256, 2), (12, 4, 2, 128, 224, 1), (27, 8, 2, 128, 256, 2), (42, 8, 2, 128, 160, 1)])
 def test_moe_slots(be, rows, E, topk, hidden, inter, ks, capfd, monkeypatch):
     """2 .. 64 rows (csrc/qgemm_skinny.hip, experts): slots by ballot, gate | up as one launch with the activation in its epilogue, down's
     partial tiles (`ks` K splits) added with the routing weights by one launch -- one to four row blocks, experts without a row,
