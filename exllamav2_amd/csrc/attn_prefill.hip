@@ -24,11 +24,11 @@
 // Bound: MFMA (2 * s * T * hd FLOP per head) -- 16 MFMAs per 32 keys per wave against ~60 VALU ops of softmax.
 #include "hw.h"
 #include "errors.h"
+#include "scratch.h"
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
-f16* prefill_scratch_try(size_t bytes, void* stream, int kind);       // qgemm_prefill.hip: scratch per (device, stream); kind 4 is this file's
 
 #ifndef FP_RPW
 #define FP_RPW 2                   // 16-row query blocks per wave: every K / V fragment read from LDS feeds FP_RPW MFMAs
@@ -427,6 +427,7 @@ int exl2_flash_prefill_ex(const void* q, const void* k_cache, const void* v_cach
     // 333 rows of a prompt's start 17.0 (three splits: 23.1), 500 rows 22.3 (four: 25.6).  Of 297 shapes (8 - 64 heads of 64, 128, 256, 4 -
     // 1024 rows behind 0 - 8000 keys) none that it splits is slower for it, one that it leaves (31.5) would gain 1.8
     a.splits = 1;
+    std::unique_lock<std::recursive_mutex> turn;             // the partial results are this call's until the merging launch
     if (!ws && !cache_seqlens)
     {
         const long wgs = (long)((q_len + FP_BQ - 1) / FP_BQ) * num_heads * batch;
@@ -441,6 +442,7 @@ int exl2_flash_prefill_ex(const void* q, const void* k_cache, const void* v_cach
             const double split = tile * (wgs * n > 256 ? 1.3 : 1.0) * ((tiles + n - 1) / n) + 2.0 + 0.5 * n + 0.45e-6 * (double)bytes;
             if (split < tile * tiles)
             {
+                turn = scratch_turn(stream);
                 a.part = (float*)prefill_scratch_try(bytes, stream, 4);
                 if (a.part) a.splits = n;
             }

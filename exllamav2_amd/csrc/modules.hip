@@ -578,6 +578,7 @@ static int moe_forward_slots(QMoEMLP* m, f16* x, const f16* xg, int rows, const 
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t b_xg = xg || !m->w1[0]->dev.perm ? 0 : up((size_t)rows * hidden * 2), b_act = up((size_t)E * 16 * rb * inter * 2),
                  b_part = (size_t)E * d.groups * d.ks * 4 * rb * 2 * 64 * sizeof(f32x4);
+    const auto turn = scratch_turn(stream);
     f16* const buf = prefill_scratch_try(b_xg + b_act + b_part, stream, 3);
     if (!buf) return 1;
     f16* const act = (f16*)((u8*)buf + b_xg);
@@ -613,6 +614,7 @@ static int moe_forward_tile(QMoEMLP* m, f16* x, int rows, void* stream)
     // the buffers one behind the other: the stage fills of a section's partial last item read up to 192 bytes past a row
     const size_t b_xg = up((size_t)chunk * hidden * 2 + 256), b_act = up(pairs * inter * 2 + 256), b_part = up(pairs * hidden * 4), b_list = up(pairs * 4),
                  b_of = up(pairs * 4), b_seg = up((size_t)(E + 1) * 4);
+    const auto turn = scratch_turn(stream);
     f16* const buf = prefill_scratch_try(b_xg + (m->tile_pair ? 1 : 2) * b_act + b_part + b_list + b_of + b_seg, stream, 3);
     if (!buf) return 1;
     u8* at = (u8*)buf;

@@ -2,6 +2,7 @@
 // 256 x 256 tiles, B decoded once per call; qgemm_prefill.hip: the row pre-pass) share with their host driver.
 #pragma once
 #include "qgemv_common.h"
+#include "scratch.h"
 
 struct PrefillArgs
 {
@@ -12,12 +13,6 @@ struct PrefillArgs
     int M, c_mode;
 };
 
-// qgemm_prefill.hip: per (device, stream) scratch that lives until exl2_release_scratch; kind 0 = staged activation rows,
-// 1 = decoded weight fragments, 2 = split-K partial tiles, 3 = a sparse block's lists and expert rows (two buffers of one call must not alias)
-int prefill_scratch(size_t bytes, void* stream, int kind, f16** out);
-// the same for a route that only wants it: null (and no error) where it cannot be had -- inside a graph capture that would grow it, out of
-// memory -- and the caller takes the route that needs none
-f16* prefill_scratch_try(size_t bytes, void* stream, int kind);
 int stage_rows_plain(const f16* a, int lda, const u16* perm, f16* out, int K, int rows, void* stream);
 
 // qgemm_skinny.hip (17 .. 128 rows): 0 = launched, 1 = does not apply (the many-row kernel takes the call), < 0 = error (message set)

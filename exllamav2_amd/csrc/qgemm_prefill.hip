@@ -160,6 +160,14 @@ f16* prefill_scratch_try(size_t bytes, void* stream, int kind)
     exl2_set_error("%s", "");
     return nullptr;
 }
+
+// (a fixed number of locks: streams come and go, two that share one only wait for a few launch calls)
+std::unique_lock<std::recursive_mutex> scratch_turn(void* stream)
+{
+    static std::recursive_mutex turns[64];
+    const size_t h = ((size_t)stream >> 4) ^ ((size_t)stream >> 12) ^ (size_t)exl2_current_device();
+    return std::unique_lock<std::recursive_mutex>(turns[h & 63]);
+}
 static int stage_scratch(size_t bytes, void* stream, f16** out) { return prefill_scratch(bytes, stream, 0, out); }
 
 // Frees the staging buffers (live and retired) of the current device: those of `stream`, or of every stream when all_streams
@@ -268,6 +276,7 @@ int qgemm_prefill_launch(GemvJob* jobs, int n_jobs, int M, bool gptq, void* stre
     // K > ~64.5 k at the default chunk).  The chunk shrinks instead of the route changing.
     while ((size_t)(chunk + 256) * (size_t)k_max * 2 >= ((size_t)1 << 31) && chunk > 256) chunk = (chunk / 2 + 255) & ~255;
     EXL2_REQUIRE((size_t)(chunk + 256) * (size_t)k_max * 2 < ((size_t)1 << 31), "prefill: K = %d is too wide for the staged-row window", k_max);
+    const auto turn = scratch_turn(stream);
     f16* stage = nullptr;
     // + 256 rows: qgemm_mfma.hip reads whole row blocks (rows >= M hold stale values, feed only rows that are never stored)
     { const int rc = stage_scratch((size_t)(chunk + 256) * k_max * 2, stream, &stage); if (rc) return rc; }

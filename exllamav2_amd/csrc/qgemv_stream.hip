@@ -24,6 +24,7 @@
 //     v_mfma_f32_16x16x32_f16, group scale applied to the fp32 partial sums (qgemv_common.h); bias / residual / MoE
 //     routing weight in the epilogue.
 #include "qgemv_common.h"
+#include "scratch.h"
 #include "errors.h"
 #include <stdio.h>
 #include <stdlib.h>
@@ -619,6 +620,7 @@ static int qgemv_phased_launch(GemvJob* jobs, int n_jobs, int M, bool gptq, int 
         if (items_max > 1) { items_max = (items_max * 3) / 4 > 0 ? (items_max * 3) / 4 : 1; continue; }
         return 1;
     }
+    const auto turn = scratch_turn(stream);
     {
         const int rc = stage_rows_for_decode(jobs, n_jobs, M, stream, args.ap, args.ap_ld);
         if (rc) return rc;

@@ -7,6 +7,7 @@
 // and spent 80 % of the test suite's time in futex calls.
 #include "hw_emu.h"
 #include <sys/mman.h>
+#include <unistd.h>
 #if !defined(__x86_64__)
 #include <ucontext.h>
 #endif
@@ -121,6 +122,8 @@ void emu_block_on(EmuBarrier* bar, unsigned gen)
 
 void emu_launch(dim3 grid, dim3 block, size_t smem, const std::function<void()>& body)
 {
+    // (EXL2_EMU_YIELD: another host thread's launch comes in behind every launch)
+    struct Yield { ~Yield() { if (getenv("EXL2_EMU_YIELD")) usleep(2000); } } yield_after_the_launch;
     std::lock_guard<std::mutex> guard(g_launch_mutex);
     if (block.y != 1 || block.z != 1 || block.x % 64 != 0 || block.x > MAX_THREADS)
     {

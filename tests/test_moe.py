@@ -244,6 +244,22 @@ def test_moe_without_scratch(be, rows, monkeypatch):
     _moe_case(be, rows, True, gate_scale=0.6, bias=0.5)
 
 
+@pytest.mark.parametrize("rows", [9, 70])
+def test_moe_threads_on_one_stream(be, rows, monkeypatch):
+    """Blocks of their own buffers, run by three host threads on one stream at the same time: the scratch between a call's launches is its own."""
+    import threading
+    from concurrent.futures import ThreadPoolExecutor
+    monkeypatch.setenv("EXL2_EMU_YIELD", "1")
+    together = threading.Barrier(3)
+
+    def run(moe, xt):
+        together.wait()
+        be.ext.q_moe_mlp_forward_(moe, xt)
+
+    with ThreadPoolExecutor(3) as pool:
+        for f in [pool.submit(_moe_case, be, rows, True, gate_scale=0.6, seed=31 + i, run=run) for i in range(3)]: f.result()
+
+
 def test_moe_model_forward(be):
     """Mixtral-style model through the ordinary ExLlamaV2 loop (config.num_experts > 0): prefill + decode run, logits are
     finite, two identical sequences in a batch produce identical rows, and the sparse MLP of layer 0 applied by hand to

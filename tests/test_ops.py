@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from oracle import modules as OM
+from tests.util import make_exl2
 
 F16 = np.float16
 
@@ -441,6 +442,45 @@ def test_flash_prefill_without_heads_is_refused(be):
     for heads in (0, -2):
         with pytest.raises(Exception, match="heads"):
             be.ext.lib.check(be.ext.lib.exl2_flash_prefill(t.data_ptr(), t.data_ptr(), t.data_ptr(), t.data_ptr(), None, None, 1, 2, heads, 1, 64, 0, 0, 10, 2, 0.125, 1, None))
+
+
+@pytest.mark.parametrize("what", ["attention", "17 rows", "130 rows", "9 rows"])
+def test_threads_that_launch_on_one_stream(be, what, monkeypatch):
+    """Calls of several launches with scratch between them (csrc/scratch.h), from four host threads on one stream: every thread reads its own
+    parts back -- the same bits as alone."""
+    import threading
+    monkeypatch.setenv("EXL2_EMU_YIELD", "1")
+    if what == "9 rows": monkeypatch.setenv("EXL2_GEMV_PHASED", "1")
+    calls, keep = [], []
+    for i in range(4):
+        rng = np.random.default_rng(i)
+        if what == "attention":
+            q, k, v = (be.t(rng.standard_normal((1, n, 2, 64)).astype(F16)) for n in (3, 400, 400))
+            out = torch.zeros((1, 3, 2, 64), dtype=torch.float16, device=be.device)
+            calls.append((lambda q=q, k=k, v=v, out=out: be.ext.flash_prefill(q, k, v, out, None, None, len_const=397, len_offset=3), out))
+        else:
+            _, _, w, h = make_exl2(be, 256, 32, [(4, 32, 256)], seed=i)
+            a = be.t(rng.standard_normal((int(what.split()[0]), 256)).astype(F16))
+            out = torch.zeros((a.shape[0], 32), dtype=torch.float16, device=be.device)
+            keep.append((w, h))
+            calls.append((lambda a=a, h=h, out=out: be.ext.gemm_half_q_half(a, h, out), out))
+    want = []
+    for f, out in calls:
+        f()
+        want.append(be.n(out).copy())
+    wrong = []
+
+    def work(i):
+        for _ in range(5):
+            calls[i][1].zero_()
+            calls[i][0]()
+            if not np.array_equal(be.n(calls[i][1]).view(np.uint16), want[i].view(np.uint16)): wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads: t.start()
+    for t in threads: t.join()
+    for _, h in keep: be.ext.free_q_matrix(h)
+    assert not wrong, wrong
 
 
 @pytest.mark.parametrize("be", [pytest.param("hip", marks=pytest.mark.gpu)], indirect=True)
