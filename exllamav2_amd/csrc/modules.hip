@@ -17,6 +17,7 @@
 #include "chain_sync.h"
 #include "moe.h"
 #include "errors.h"
+#include <math.h>
 #include <string.h>
 #include <stdlib.h>
 #include <stdio.h>
@@ -600,6 +601,20 @@ static int moe_forward_slots(QMoEMLP* m, f16* x, const f16* xg, int rows, const 
     return EXL2_OK;
 }
 
+// 2 .. 16 rows: the grouped launches instead.  The slots route has a launch more and takes almost as long for one expert as for all; the grouped
+// launches grow with the experts that have rows (E (1 - (1 - k / E)^rows) where the router spreads evenly) and a little with the rows.  Whole blocks,
+// weights from memory, us, grouped | slots: 8 GPTQ experts of 4096 x 14336, one each, 2 / 4 / 5 rows 62 | 97, 105 | 116, 117 | 118, two each,
+// 2 / 3 rows 99 | 118, 132 | 129; EXL2 4 experts of 512 x 1024, two each, 2 / 8 / 14 rows 20.2 | 25.0, 22.8 | 25.4, 25.4 | 25.6; 8 of 2048 x 1024,
+// one each, 3 / 5 rows 30.3 | 35.2, 36.9 | 36.0; 4096 x 14336, two each, 2 rows 123 | 103
+static bool moe_grouped_wins(const QMoEMLP* m, int rows)
+{
+    const float E = (float)m->num_experts;
+    const float chosen = E * (1.0f - powf(1.0f - (float)m->num_experts_per_token / E, (float)rows));
+    const long long weights = (long long)m->hidden * m->w1[0]->width;
+    const float limit = m->w1[0]->is_gptq ? 4.1f : weights <= (1 << 19) ? 6.0f : weights <= (1 << 21) ? 4.1f : 3.2f;
+    return rows <= 16 && chosen + (float)rows / 6.0f < limit && !ENV_SET("EXL2_SKINNY_EXPERT_KS");      // (a forced number of splits asks for the slots)
+}
+
 // norm and router have run (temp_state: normalised rows, temp_logits: routing weights).  Passes of at most MOE_TILE_ROWS rows bound
 // the scratch (8x7B: 0.37 GB).  0 = done, 1 = does not apply (or its scratch cannot be had)
 #define MOE_TILE_ROWS 4096
@@ -803,13 +818,15 @@ static int moe_forward(void* handle, void* x_, int rows, const MoeChainOut& co, 
     };
     // ---- 2 .. 64 rows: every expert's rows by a ballot over the routing weights, gate | up as one launch, down's partial tiles as one, one that
     // adds splits and experts (qgemm_skinny.hip)
-    if (rows >= 2 && rows <= 64 && m->tile_ok && m->tile_pair && !ENV_SET("EXL2_MOE_SERIAL") && !ENV_SET("EXL2_MOE_NO_GROUP"))
+    const bool slots = rows >= 2 && rows <= 64 && m->tile_ok && m->tile_pair && !ENV_SET("EXL2_MOE_SERIAL") && !ENV_SET("EXL2_MOE_NO_GROUP");
+    const bool few = slots && moe_grouped_wins(m, rows);
+    if (slots && !few)
     {
         const int rc = moe_forward_slots(m, x, have_xg ? xg : nullptr, rows, co, npart_out, stream);
         if (rc <= 0) return rc;
     }
-    // ---- gate and up cut into different sections: grouped route (rows <= 16): all experts' gate|up in ONE launch (SiLU * up in the epilogue,
-    // written in each down projection's packed order), all experts' down in ONE launch (weighted partial outputs), one combine.  Replaces the
+    // ---- gate and up cut into different sections, or few experts chosen: grouped route (rows <= 16): all experts' gate|up in ONE launch (SiLU * up
+    // in the epilogue, written in each down projection's packed order), all experts' down in ONE launch (weighted partial outputs), one combine.  Replaces the
     // per-expert launch loop below (3 launches per expert: q_mlp.cu:318-402 has the same shape, moe_mlp.py:255-323 a
     // Python loop above 4 rows).
     if (m->group_ok && rows <= MAX_GEMV_ROWS && 2 * MAX_GEMV_ROWS <= m->max_rows && (long long)E * rows <= m->max_rows &&
@@ -849,6 +866,11 @@ static int moe_forward(void* handle, void* x_, int rows, const MoeChainOut& co, 
             // (the gate|up launch wrote only temp_a: the serial route below recomputes everything)
         }
         else if (rc < 0) EXL2_FAIL(EXL2_E_INVALID, "q_moe_mlp_forward_: grouped gate|up launch rejected (%d)", rc);
+    }
+    if (few)
+    {
+        const int rc = moe_forward_slots(m, x, have_xg ? xg : nullptr, rows, co, npart_out, stream);
+        if (rc <= 0) return rc;
     }
     // ---- batched route (round 5; rows <= 16 the grouped launch declined: Mixtral's 16 x 14336 down_proj rows do not fit its LDS):
     // the experts on the streaming / phased kernels like the serial loop below, but (1) gate and up read the rows gathered ONCE into

@@ -187,6 +187,7 @@ def test_moe_experts_with_biases_launch_by_launch(be, rows, shared_perm, env, mo
 def test_moe_gptq_and_gelu_experts(be, rows, tile_rb, route, gptq, gelu, capfd, monkeypatch):
     """GPTQ experts (zero points beside the scales) and GELU units in the kernels that run all experts in one launch, at every number of row blocks"""
     monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    monkeypatch.setenv("EXL2_SKINNY_EXPERT_KS", "1")
     if tile_rb: monkeypatch.setenv("EXL2_TILE_RB", str(tile_rb))
     _moe_case(be, rows, True, E=4, hidden=128, inter=288, gate_scale=0.6, max_rows=160, gptq=gptq, gelu=gelu, bias=0.5, spec_dn=[(5, 32, 64), (3, 32, 224)])
     assert f"route: {route}" in capfd.readouterr().err
@@ -208,6 +209,7 @@ def test_moe_slots_publish_for_the_next_consumer(be, rows, hidden, tiled, capfd,
     """The slots route inside a chained step: its last launch leaves x times the next consumer's norm weight in that consumer's order (plain and
     tiled) and the partial sums of squares of every row, one per workgroup."""
     monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    monkeypatch.setenv("EXL2_SKINNY_EXPERT_KS", "1")
     rng = np.random.default_rng(71)
     inv = rng.permutation(hidden).astype(np.uint16)
     norm = (1.0 + 0.2 * rng.standard_normal(hidden)).astype(F16)
@@ -241,7 +243,18 @@ def test_moe_without_scratch(be, rows, monkeypatch):
     """Scratch that cannot be had (as inside a capture on a stream that holds none): the routes that need none answer."""
     be.ext.release_scratch()
     monkeypatch.setenv("EXL2_EMU_CAPTURING", "1")
+    monkeypatch.setenv("EXL2_SKINNY_EXPERT_KS", "1")
     _moe_case(be, rows, True, gate_scale=0.6, bias=0.5)
+
+
+@pytest.mark.parametrize("rows,E,topk,hidden,inter,gptq,route", [
+    (2, 8, 2, 128, 256, 0, "grouped"), (3, 8, 2, 128, 256, 0, "grouped"), (4, 8, 2, 128, 256, 0, "slots"), (12, 4, 2, 128, 256, 0, "grouped"), (13, 4, 2, 128, 256, 0, "slots"),
+    (3, 4, 2, 128, 4128, 0, "grouped"), (4, 4, 2, 128, 4128, 0, "slots"), (2, 4, 2, 512, 4128, 0, "slots"), (3, 4, 2, 128, 256, 32, "grouped"), (4, 4, 2, 128, 256, 32, "slots")])
+def test_moe_grouped_or_slots(be, rows, E, topk, hidden, inter, gptq, route, capfd, monkeypatch):
+    """2 rows on: the grouped launches while few experts are chosen, by the experts' sizes, on both sides of every line."""
+    monkeypatch.setenv("EXL2_DEBUG_ROUTE", "1")
+    _moe_case(be, rows, True, E=E, topk=topk, hidden=hidden, inter=inter, gate_scale=0.6, gptq=gptq)
+    assert f"route: {route} rows={rows} " in capfd.readouterr().err
 
 
 @pytest.mark.parametrize("rows", [9, 70])
