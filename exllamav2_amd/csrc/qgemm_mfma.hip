@@ -604,27 +604,53 @@ int qgemm_mfma_launch(const PrefillArgs* pas, int n, bool gptq, void* stream)
         for (int i = 0; i < n; i++) { const int rc = qgemm_mfma_launch(pas + i, 1, gptq, stream); if (rc) return rc; }
         return EXL2_OK;
     };
-    // (many rounds anyway: a launch per matrix keeps one matrix' fragments in the memory-side cache, 0.2 % at 16384 rows.  A matrix of more
-    // sections than the arguments name can neither split K nor have its fragments made: the others are not held to that)
-    if (n > 1 && ((long)blocks * ((M + 255) / 256) >= 8L * cus || (!runs && supers_max > 0))) return one_by_one();
-    int mt = 8, ks = 1;
+    // best tile height (mt x 32 rows) and K splits of `nb` column blocks with `items` super-chunks, and what they take
+    struct Choice { int mt, ks; double t; };
+    auto choose = [&](int nb, int items) -> Choice
     {
-        const double steps = 2.0 * (supers_max > 0 ? supers_max : (K + SUPER_ROWS - 1) / SUPER_ROWS);
-        double best = 0.0;
+        const double steps = 2.0 * (items > 0 ? items : (K + SUPER_ROWS - 1) / SUPER_ROWS);
+        Choice best = {8, 1, 0.0};
         for (int c = 0; c < 2; c++)
         {
             const int mm = c ? 4 : 8;
-            const long tiles = (long)blocks * ((M + 32 * mm - 1) / (32 * mm));
+            const long tiles = (long)nb * ((M + 32 * mm - 1) / (32 * mm));
             for (int k = 1; k <= 8; k++)
             {
                 if (k > 1 && (!runs || tiles * k > cus || steps / k < 8.0)) break;
                 const long rounds = (tiles * k + cus - 1) / cus;
                 const double full = tiles * k > cus ? 1.0 : 0.0;
                 const double t = rounds * (steps / k) * (mm == 8 ? 1.19 + 0.17 * full : 0.80 + 0.03 * full) + (k > 1 ? 5.0 + tiles * k * mm * 0.0164 : 0.0);
-                if (best == 0.0 || t < best) { best = t; mt = mm; ks = k; }
+                if (best.t == 0.0 || t < best.t) best = {mm, k, t};
             }
         }
+        return best;
+    };
+    const Choice all = choose(blocks, supers_max);
+    // Several matrices: one launch, or one each?  Many rounds anyway: each keeps one matrix' fragments in the memory-side cache (0.2 % at 16384
+    // rows).  A matrix of more sections than the arguments name can neither split K nor have its fragments made: the others are not held to
+    // that.  Otherwise by the estimates: a launch more is about 10 us, and fragments that do not stay in the cache (256 MB; with the
+    // rows and the results) until they are read cost 0.27 us per MB.  Whole MLPs, one launch | one each, us: 4096 x 11008 333 rows 220 | 240,
+    // 1024: 392 | 373, 1408: 504 | 466, 1664: 536 | 587; 4096 x 14336 256 rows 243 | 225, 704: 421 | 375, 1664: 761 | 654; 5120 x 13824 576 rows
+    // 526 | 446, 1100: 725 | 618, 1280: 699 | 727; 8192 x 28672 256 rows 766 | 887, 640: 1390 | 1781
+    if (n > 1)
+    {
+        bool apart = (long)blocks * ((M + 255) / 256) >= 8L * cus || (!runs && supers_max > 0);
+        if (!apart && runs)
+        {
+            double t_all = all.t, t_each = 10.0 * (n - 1), frag_mb = 0.0, io_mb = (double)M * K * 2e-6;
+            auto cold = [&](double frag, double io) { return frag + io > 225.0 ? 0.27 * frag : 0.0; };
+            for (int i = 0; i < n; i++)
+            {
+                const double frag = (double)p.job[i].m.N * K * 2e-6, io = (double)M * p.job[i].m.N * 2e-6;
+                t_each += choose((p.job[i].m.N + MF_BN - 1) / MF_BN, supers[i]).t + cold(frag, io + (double)M * K * 2e-6);
+                frag_mb += frag; io_mb += io;
+            }
+            t_all += cold(frag_mb, io_mb);
+            apart = t_each < t_all;
+        }
+        if (apart) return one_by_one();
     }
+    int mt = all.mt, ks = all.ks;
     if (const char* e = getenv("EXL2_PREFILL_MT")) { const int v = atoi(e); if (v == 4 || v == 8) { mt = v; ks = 1; } }
     if (const char* e = getenv("EXL2_PREFILL_KS")) { const int v = atoi(e); if (v >= 1 && v <= 16 && runs && v <= supers_max) ks = v; }
     if (ks > 1)

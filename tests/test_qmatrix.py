@@ -314,6 +314,42 @@ def test_splits_and_fragments_without_scratch(be, m, ks_env, pre_env, capfd, mon
     be.ext.free_q_matrix(h)
 
 
+@pytest.mark.parametrize("be", [pytest.param("hip", marks=pytest.mark.gpu)], indirect=True)
+@pytest.mark.parametrize("k,n,m,launches", [(4096, 8192, 333, 1), (4096, 11008, 333, 1), (4096, 11008, 1024, 2), (4096, 14336, 160, 2)])
+def test_prefill_gate_and_up_together_or_apart(be, k, n, m, launches, capfd, monkeypatch):
+    """gate | up of many rows in one launch, or one each where the fragments of both do not stay in the cache: the route, and the result against
+    the float32 product of the fp16 weights (fp16 steps of gate, up and their product: 2^-11 each, a quarter more for their sums' roundings)."""
+    from exllamav2_amd.ext import none_tensor
+    from exllamav2_amd.synth import synth_linear
+    monkeypatch.setenv("EXL2_PREFILL_TRACE", "1")
+    g = torch.Generator(device=be.device)
+    g.manual_seed(n + m)
+    w1 = synth_linear(k, n, ([5, 4], [0.1, 0.9], 128), be.device, g)
+    w3 = synth_linear(k, n, ([5, 4], [0.1, 0.9], 128), be.device, g, invperm=w1["q_invperm"])
+    w2 = synth_linear(n, k, ([4], [1.0], 128), be.device, g)
+    h = [be.ext.make_q_matrix_from_dict(w, none_tensor) for w in (w1, w3, w2)]
+    ta, tb = (torch.empty((m, n), dtype=torch.float16, device=be.device) for _ in range(2))
+    ts = torch.empty((m, k), dtype=torch.float16, device=be.device)
+    norm = torch.ones((k,), dtype=torch.float16, device=be.device)
+    mlp = be.ext.make_q_mlp(norm, none_tensor, True, 1e-5, *h, ts, ta, tb, none_tensor, m, False, True, none_tensor, none_tensor, False, False)
+    x = torch.randn((m, k), generator=g, device=be.device).half()
+    y = x.clone()
+    be.ext.q_mlp_forward_(mlp, y)
+    assert sum(f" K={k} " in line for line in capfd.readouterr().err.splitlines()) == launches
+    dense = []
+    for hh, (a, b) in zip(h, ((k, n), (k, n), (n, k))):
+        dense.append(torch.empty((a, b), dtype=torch.float16, device=be.device))
+        be.ext.reconstruct(hh, dense[-1])
+    xf = x.float()
+    xn = (xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + 1e-5)).half().float()
+    want = (torch.nn.functional.silu(xn @ dense[0].float()) * (xn @ dense[1].float())) @ dense[2].float()
+    err = (y.float() - xf - want).norm() / want.norm()
+    # (x + delta leaves as fp16: half a step of x's size beside delta's own)
+    assert err <= 1.25 * 3 * 2.0 ** -11 + 2.0 ** -11 * (y.float().norm() / want.norm())
+    be.ext.free_q_mlp(mlp)
+    for hh in h: be.ext.free_q_matrix(hh)
+
+
 def test_prefill_matrix_of_many_sections_beside_one_of_few(be, capfd, monkeypatch):
     """gate in one section, up in more than a kernel's argument block names: up decodes inside its product, gate's weights are decoded ahead as
     they are alone -- the two do not share a launch."""
