@@ -725,7 +725,7 @@ int exl2_free_q_moe_mlp(void* handle)
 
 // q_moe_mlp_forward_ (ext_qmlp.cpp:245-272 -> QMoEMLP::forward_, q_mlp.cu:318-402): in place on x [rows, hidden].
 // The reference takes rows <= 4; here any row count.  One row: the lean kernels over the chosen experts.  2 .. 64: moe_forward_slots, all
-// experts over the rows that chose them.  More: moe_forward_tile, over lists of them (1093 rows of a 4096 x 14336 x 8 block: 1.15 ms, in
+// experts over the rows that chose them (the grouped launches where those are few: moe_grouped_wins).  More: moe_forward_tile, over lists of them (1093 rows of a 4096 x 14336 x 8 block: 1.15 ms, in
 // passes of 16 rows 43 ms).  Experts whose gate and up are cut into different sections: the grouped launches up to 16 rows, moe_forward_tile
 // from 17 on.  Experts that share no packed order, or scratch that cannot be had: the routes at the end, 16 rows at a time.
 static int moe_forward(void* handle, void* x_, int rows, const MoeChainOut& co, int* npart_out, void* stream)
